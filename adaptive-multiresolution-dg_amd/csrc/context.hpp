@@ -299,6 +299,30 @@ class Context {
   FusedPlan& fused_plan(const StageProblem& p);
   template <class T>
   void stage_body(const StageProblem& p, FusedPlan& pl, int scheme, int stage, double dt);
+  // The stage on source lists (list.hpp), the form that runs unless the caller
+  // fixed a mapping for one of its kernel classes: list_stage.hip.
+  struct ListPlan;
+  std::shared_ptr<ListPlan> list_plan;
+  bool list_stage_fits() const;
+  ListPlan& get_list_plan(const StageProblem& p);
+  template <class T>
+  void stage_list(const StageProblem& p, int scheme, int stage, double dt);
+  template <class T>
+  void flux_herm(const T* up, T* fp, int kind, T s, int ncomp);
+  // lists of the given kinds for the current grid, level-sum cap and
+  // interpolation family (nz: which table blocks count, default nz_tab)
+  void ensure_lists(int kind0, int nkind, const uint8_t* nz);
+  void list_nonzero_tables();
+  static constexpr int kListKinds = 4;
+  DevBuf<uint8_t> nz_tab;
+  int nz_interp = -1;
+  DevBuf<int4> l_meta[kListKinds * kMaxDim];
+  DevBuf<int2> l_ent[kListKinds * kMaxDim];
+  DevBuf<int32_t> l_total;
+  int64_t list_version[kListKinds] = {-1, -1, -1, -1};
+  int list_level_cap[kListKinds] = {-1, -1, -1, -1}, list_interp[kListKinds] = {-1, -1, -1, -1};
+  DevBuf<double> list_tmp;
+  int64_t list_ecap = 0;  // elements the phase buffers have room for
   // How a fused stage is launched: 0 one launch per phase (thread mappings
   // chosen by the autotuner), 1 one persistent cooperative launch per stage
   // (fiber tiles of 64 elements, four rest indices per thread; Lagrange family)

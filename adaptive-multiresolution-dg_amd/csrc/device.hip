@@ -21,6 +21,7 @@
 #include "context.hpp"
 #include "fiber.hpp"
 #include "kern.hpp"
+#include "list.hpp"
 #include "surplus_dev.hpp"
 #include "tile.hpp"
 #include "coop.hpp"
@@ -606,7 +607,7 @@ void Context::set_interpolation(int family) {
   t_wt.swap(alt_wt);
   t_anc_slot.swap(alt_anc_slot);
   t_anc_point.swap(alt_anc_point);
-  interp = family;
+  interp = family;  // (the source lists of the point and flux tables follow: ensure_lists)
 }
 
 struct Context::FusedPlan {
@@ -1500,11 +1501,26 @@ void Context::stage_fused(const StageProblem& p, int scheme, int stage, double d
     up32.ensure(e * P);
     for (DevBuf<float>* b : {&fp32, &fucoe32, &interA32, &interB32}) b->ensure(e * P * D);
   }
+  bool fixed = kernel_variant >= 0 || stage_launch == 1;
+  for (int c = 0; c < 4; ++c) fixed = fixed || class_variant[c + (precision == 1 ? 4 : 0)] >= 0;
+  if (!fixed && list_stage_fits()) {
+    ++stage_count;
+    if (precision == 1) stage_list<float>(p, scheme, stage, dt);
+    else stage_list<double>(p, scheme, stage, dt);
+    return;
+  }
   FusedPlan& pl = fused_plan(p);
   ++stage_count;
   if (precision == 1) stage_body<float>(p, pl, scheme, stage, dt);
   else stage_body<double>(p, pl, scheme, stage, dt);
 }
+
+template <class T>
+void Context::flux_herm(const T* upp, T* fpp, int kind, T s, int ncomp) {
+  hipLaunchKernelGGL(k_flux_herm<T>, dim3(nblocks(E() * P)), dim3(kBlock), 0, stream, upp, fpp, E(), D, kind, s, ncomp);
+}
+template void Context::flux_herm<double>(const double*, double*, int, double, int);
+template void Context::flux_herm<float>(const float*, float*, int, float, int);
 
 // One fused stage with intermediates stored in T (double, or float with split
 // tables).  Every kernel class runs one of the mappings: 0..3 per-element
@@ -1634,8 +1650,7 @@ void Context::stage_body(const StageProblem& p, FusedPlan& pl, int scheme, int s
       }
     });
     if (interp == 1) {
-      hipLaunchKernelGGL(k_flux_herm<T>, dim3(nblocks(E() * P)), dim3(kBlock), 0, stream, upp, fpp, E(), D,
-                         p.flux_kind, T(p.flux_param), ncomp);
+      flux_herm<T>(upp, fpp, p.flux_kind, T(p.flux_param), ncomp);
       ++stage_launches;
     }
     prof_end();
@@ -1712,6 +1727,8 @@ std::vector<uintptr_t> Context::step_key(const StageProblem& p, int scheme, int 
       static_cast<uintptr_t>(nstage), static_cast<uintptr_t>(p.flux_kind), bits(p.flux_param),
       static_cast<uintptr_t>(use_inst_dt), use_inst_dt ? ptr(d_inst_dt.p) : bits(dt), inst_alpha.size()};
   for (int d = 0; d < D; ++d) key.push_back(bits(p.alpha[d]));
+  for (int64_t v : list_version) key.push_back(static_cast<uintptr_t>(v));
+  key.insert(key.end(), {ptr(list_plan.get()), ptr(list_tmp.p)});
   if (key[kKeyU] != ptr(u.p) || key[kKeyUNext] != ptr(u_next.p)) throw std::logic_error("step key layout");
   return key;
 }

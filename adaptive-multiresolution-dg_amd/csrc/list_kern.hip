@@ -1,0 +1,457 @@
+// Source lists of the fibers and the sweeps that run on them; see list.hpp.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <climits>
+#include <stdexcept>
+
+#include "list.hpp"
+
+namespace adg {
+namespace {
+
+constexpr int kBlock = 256;
+constexpr int kWave = 64;
+
+inline unsigned nblocks(int64_t n) { return static_cast<unsigned>((n + kBlock - 1) / kBlock); }
+
+// ---------------------------------------------------------------------------
+// build
+
+__global__ __launch_bounds__(kBlock) void k_list_nz(uint8_t* nz, const double* M, int64_t n, int block, int bit,
+                                                    int clear) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  bool any = M == nullptr;
+  if (M)
+    for (int j = 0; j < block; ++j) any = any || M[i * block + j] != 0.;
+  uint8_t v = nz[i];
+  if (clear) v &= static_cast<uint8_t>(~bit);
+  nz[i] = any ? static_cast<uint8_t>(v | bit) : v;
+}
+
+__global__ void k_list_zero(int32_t* p, int n) {
+  if (static_cast<int>(threadIdx.x) < n) p[threadIdx.x] = 0;
+}
+
+// Present sources of element e along dimension d for the lists of one kind,
+// ascending: f(source element, source slot).
+template <class F>
+__device__ __forceinline__ void list_sources(const ListBuildArgs& a, int kind, int d, int64_t e, int st, F&& f) {
+  const int fb = a.fbase[d][e];
+  int maxl = a.fmaxl[d][e];
+  if (a.level_cap >= 0) {  // coarse grid (FastMultiplyLU::transform_1D_coarse_grid)
+    const int ls = a.lsum[e];
+    if (ls > a.level_cap) return;
+    maxl = min(maxl, a.level_cap - ls + slot_level(st));
+  }
+  const int32_t* fmap = a.fmap[d];
+  const uint8_t* nz = a.nz + static_cast<int64_t>(st) * a.ns;
+  const bool flx = kind == LIST_FLX || kind == LIST_LIN;
+  for_each_present(st, maxl, flx, LU_FULL, a.fbits[d], fb, [&](int s) {
+    if (!(nz[s] >> kind & 1)) return;
+    const int src = fmap[fb + s];
+    if (src >= 0) f(src, s);
+  });
+}
+
+// Thread per (kind, dimension, target): counts its sources, takes room for
+// the block's sources with one atomic add, and writes them.  Where a target's
+// entries lie differs from run to run, what they hold does not.
+__global__ __launch_bounds__(kBlock) void k_list_build(ListBuildArgs a, int kind0) {
+  __shared__ int s_wave[kBlock / kWave];
+  __shared__ int s_base;
+  const int kind = kind0 + static_cast<int>(blockIdx.y) / a.D, d = static_cast<int>(blockIdx.y) % a.D;
+  const int list = kind * a.D + d;
+  const int64_t e = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  int n = 0, nu = 0, st = 0;
+  if (e < a.E) {
+    st = a.slot[d][e];
+    const int lt = slot_level(st);
+    list_sources(a, kind, d, e, st, [&](int, int s) {
+      ++n;
+      nu += slot_level(s) <= lt;
+    });
+  }
+  int inc = n;  // inclusive sum over the wavefront
+  for (int o = 1; o < kWave; o <<= 1) {
+    const int v = __shfl_up(inc, o);
+    if (lane >= o) inc += v;
+  }
+  if (lane == kWave - 1) s_wave[wave] = inc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int sum = 0;
+    for (int w = 0; w < kBlock / kWave; ++w) {
+      const int v = s_wave[w];
+      s_wave[w] = sum;
+      sum += v;
+    }
+    s_base = atomicAdd(&a.total[list], sum);
+  }
+  __syncthreads();
+  if (e >= a.E) return;
+  int beg = s_base + s_wave[wave] + inc - n;
+  if (static_cast<int64_t>(beg) + n > a.cap[list]) {  // (the bound of the host is exceeded: never)
+    atomicOr(a.err, ERR_COOP);
+    a.meta[list][e] = make_int4(0, 0, st, a.inst[e]);
+    return;
+  }
+  a.meta[list][e] = make_int4(beg, nu | n << 16, st, a.inst[e]);
+  int2* ent = a.ent[list];
+  list_sources(a, kind, d, e, st, [&](int src, int s) { ent[beg++] = make_int2(src, s); });
+}
+
+// ---------------------------------------------------------------------------
+// sweeps
+//
+// A thread evaluates one rest index of a target (the PT outputs of the swept
+// dimension): per source it reads an 8-byte entry, the PF values of the source
+// and its PF*PT table block.  Bound: the vector memory unit, which takes a
+// wavefront's load of 16 bytes per lane in 16 cycles or more (measured busy 73
+// to 74 % of the time; table loads and value loads cost about a third of the
+// kernel each).  Wider tiles of rest indices per thread (2, 4) save table
+// loads but scatter the value loads and lose wavefronts: no faster; staging
+// the table blocks in LDS was 1.2 to 3 times slower (rounds of copies for
+// lists of 3 to 5 sources).  256 3D instances, 213 thousand elements, k = 2,
+// m = 3: phases 1597 us per launch of 12 and 20 sweeps (the walks they
+// replace: 2.3 ms), last sweeps 1950 us (2.9 ms with their sums).
+
+// Loads through the global address space at a uniform base plus a 32-bit byte
+// offset (list_stage_fits() keeps every array a sweep reads below 4 GiB).
+template <class T>
+__device__ __forceinline__ T gl(const void* base, uint32_t bytes, int i = 0) {
+  return ((const __attribute__((address_space(1))) T*)((const __attribute__((address_space(1))) char*)base + bytes))[i];
+}
+typedef int vi2 __attribute__((ext_vector_type(2)));
+typedef int vi4 __attribute__((ext_vector_type(4)));
+
+// Input and table of a term for values of type T.  x[k]: values k of a source
+// (the swept dimension has stride sdd) at the offset of its element and rest
+// index; m: the N values of the table block of (target slot, source slot).
+template <class T, int PF>
+struct ListIn;
+template <int PF>
+struct ListIn<double, PF> {
+  const double* x[PF];
+  const double* m;
+  __device__ __forceinline__ ListIn(const ListTerm& t, const double* u, int64_t E) : m(t.M) {
+    const double* b = (t.in ? t.in : u) + t.comp * (E * t.comp_size);
+    for (int k = 0; k < PF; ++k) x[k] = b + k * t.sdd;
+  }
+  __device__ __forceinline__ void values(uint32_t at, double (&v)[PF]) const {
+#pragma unroll
+    for (int k = 0; k < PF; ++k) v[k] = gl<double>(x[k], at * 8);
+  }
+  template <int N>
+  struct Block { double w[N]; };
+  template <int N>
+  __device__ __forceinline__ Block<N> block(uint32_t at) const {
+    Block<N> b;
+#pragma unroll
+    for (int i = 0; i < N; ++i) b.w[i] = gl<double>(m, at * 8, i);
+    return b;
+  }
+  template <int N>
+  static __device__ __forceinline__ void madd(double& acc, double v, const Block<N>& b, int j) { acc += v * b.w[j]; }
+};
+template <int PF>
+struct ListIn<float, PF> {
+  const double* x[PF];
+  const float* x32[PF];
+  const float *mh, *ml;
+  bool f32;
+  __device__ __forceinline__ ListIn(const ListTerm& t, const double* u, int64_t E) : mh(t.Mh), ml(t.Ml), f32(t.in32) {
+    const double* b = (t.in ? t.in : u) + t.comp * (E * t.comp_size);
+    const float* b32 = t.in32 + t.comp * (E * t.comp_size);
+    for (int k = 0; k < PF; ++k) {
+      x[k] = b + k * t.sdd;
+      x32[k] = b32 + k * t.sdd;
+    }
+  }
+  __device__ __forceinline__ void values(uint32_t at, float (&v)[PF]) const {
+#pragma unroll
+    for (int k = 0; k < PF; ++k) v[k] = f32 ? gl<float>(x32[k], at * 4) : static_cast<float>(gl<double>(x[k], at * 8));
+  }
+  template <int N>
+  struct Block { float h[N], l[N]; };
+  template <int N>
+  __device__ __forceinline__ Block<N> block(uint32_t at) const {
+    Block<N> b;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      b.h[i] = gl<float>(mh, at * 4, i);
+      b.l[i] = gl<float>(ml, at * 4, i);
+    }
+    return b;
+  }
+  template <int N>
+  static __device__ __forceinline__ void madd(float& acc, float v, const Block<N>& b, int j) {
+    acc = fmaf(v, b.l[j], acc);
+    acc = fmaf(v, b.h[j], acc);
+  }
+};
+
+// acc[i] = sum over the sources of a target, ascending, k inner, of
+// in[source][bin + k*sdd] * M(k, i).  NB sources are requested together.
+template <int PF, int PT, class T, int NB>
+__device__ __forceinline__ void list_sum(const ListTerm& t, const ListIn<T, PF>& src, const vi4 meta, uint32_t bin,
+                                         T (&acc)[PT]) {
+  constexpr int N = PF * PT;
+#pragma unroll
+  for (int i = 0; i < PT; ++i) acc[i] = T(0);
+  const uint32_t nu = meta.y & 0xffff, na = static_cast<uint32_t>(meta.y) >> 16;
+  const uint32_t lo = t.lu == LU_L ? nu : 0, hi = t.lu == LU_U ? nu : na;
+  const uint32_t Mst = __umul24(meta.z, t.ns) * N;
+  const uint32_t Tin = t.Tin;
+  const uint32_t end = (meta.x + hi) * 8;
+  for (uint32_t i = (meta.x + lo) * 8; i < end; i += 8 * NB) {
+    vi2 en[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) en[j] = gl<vi2>(t.ent, j == 0 ? i : min(i + 8 * j, end - 8));
+    typename ListIn<T, PF>::template Block<N> m[NB];
+    T x[NB][PF];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      m[j] = src.template block<N>(Mst + en[j].y * N);
+      src.values(__umul24(en[j].x, Tin) + bin, x[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+      if (j == 0 || i + 8 * j < end) {
+#pragma unroll
+        for (int q = 0; q < PT; ++q)
+#pragma unroll
+          for (int k = 0; k < PF; ++k) ListIn<T, PF>::template madd<N>(acc[q], x[j][k], m[j], k * PT + q);
+      }
+  }
+}
+
+// Term t for rest index c of element e, to out (the element's values).
+template <int PF, int PT, class T, int NB, class O>
+__device__ __forceinline__ void list_item(const ListTerm& t, const ListIn<T, PF>& src, uint32_t e, uint32_t c, O* out) {
+  const vi4 meta = gl<vi4>(t.meta, e * 16);
+  const vi2 o = gl<vi2>(t.rofs, c * 8);
+  T acc[PT];
+  list_sum<PF, PT, T, NB>(t, src, meta, o.x, acc);
+  const T cf = T(t.coef_inst ? gl<double>(t.coef_inst, meta.w * 8) : t.coef);
+  const int sod = t.sod;
+#pragma unroll
+  for (int i = 0; i < PT; ++i) out[o.y + i * sod] = O(acc[i] * cf);
+}
+
+// Sweeps of one phase: thread per (element, rest index), a row of blocks per
+// term.
+template <int PF, int PT, class T, int NB>
+__global__ __launch_bounds__(kBlock) void k_list_phase(const ListTerm* terms, uint32_t E, uint32_t R, const double* u) {
+  const ListTerm& t = terms[blockIdx.y];
+  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+  const uint32_t e = i / R, c = i - e * R;
+  if (e >= E) return;
+  const ListIn<T, PF> src(t, u, E);
+  list_item<PF, PT, T, NB>(t, src, e, c, static_cast<T*>(t.out) + static_cast<int64_t>(e) * t.Tout);
+}
+
+// Last sweep of every eval_up partial sum, added in order into the point
+// value, and the point flux.  A block holds EB elements; each of its
+// wavefronts takes every W-th term for all of them.
+template <int PF, int PT, class T, int NB>
+__global__ __launch_bounds__(512) void k_list_up_final(const ListTerm* terms, int nterm, int EB, int nch, int64_t E,
+                                                        int P, const double* u, T* up, T* fp, const double* vcoef,
+                                                        int kind, double s, int ncomp) {
+  extern __shared__ double vals[];  // [nterm][EB][P]
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), W = blockDim.x / kWave;
+  const int lane = threadIdx.x % kWave;
+  const int64_t e0 = static_cast<int64_t>(xcd_block()) * EB;
+  const int ne = static_cast<int>(min(static_cast<int64_t>(EB), E - e0));
+  for (int t = wave; t < nterm; t += W) {
+    const ListIn<T, PF> src(terms[t], u, E);
+    for (int it = lane; it < ne * nch; it += kWave) {
+      const int el = it / nch, c = it - el * nch;
+      list_item<PF, PT, T, NB>(terms[t], src, static_cast<uint32_t>(e0) + el, c, vals + (t * EB + el) * P);
+    }
+  }
+  __syncthreads();
+  const int64_t n = E * P;
+  for (int o = threadIdx.x; o < ne * P; o += blockDim.x) {
+    double v = 0.;
+    for (int j = 0; j < nterm; ++j) v += vals[j * EB * P + o];
+    const int64_t gid = e0 * P + o;
+    const T uu = T(v);
+    up[gid] = uu;
+    flux_point<T>(kind, uu, s, vcoef, fp, gid, n, ncomp);
+  }
+}
+
+// Last sweep of every right-hand-side partial sum and the penalty sweeps,
+// added in order, then the RK stage update.  Blocks as above.
+template <int PFM, int PFK, class T, int NB>
+__global__ __launch_bounds__(512) void k_list_rhs_final(const ListTerm* terms, int nterm, int npen, int EB, int nch,
+                                                         int64_t E, int K, double* rhs, const double* u,
+                                                         const double* tn, double* u_next, int scheme, int stage,
+                                                         double dt, const double* dtv, int32_t* err) {
+  extern __shared__ double vals[];  // [nterm + npen][EB][K]
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), W = blockDim.x / kWave;
+  const int lane = threadIdx.x % kWave;
+  const int64_t e0 = static_cast<int64_t>(xcd_block()) * EB;
+  const int ne = static_cast<int>(min(static_cast<int64_t>(EB), E - e0));
+  for (int t = wave; t < nterm + npen; t += W) {
+    for (int it = lane; it < ne * nch; it += kWave) {
+      const int el = it / nch, c = it - el * nch;
+      double* out = vals + (t * EB + el) * K;
+      if (t < nterm)
+        list_item<PFM, PFK, T, NB>(terms[t], ListIn<T, PFM>(terms[t], u, E), static_cast<uint32_t>(e0) + el, c, out);
+      else
+        list_item<PFK, PFK, double, NB>(terms[t], ListIn<double, PFK>(terms[t], u, E), static_cast<uint32_t>(e0) + el, c, out);
+    }
+  }
+  __syncthreads();
+  const int4* meta = terms[0].meta;
+  for (int o = threadIdx.x; o < ne * K; o += blockDim.x) {
+    double r = 0.;
+    for (int j = 0; j < nterm + npen; ++j) r += vals[j * EB * K + o];
+    const int64_t gid = e0 * K + o;
+    rhs[gid] = r;
+    const double dte = dtv ? dtv[meta[e0 + o / K].w] : dt;
+    const double un = rk_combine(scheme, stage, dte, tn[gid], u[gid], r);
+    u_next[gid] = un;
+    if (!isfinite(un)) atomicOr(err, ERR_NONFINITE);
+  }
+}
+
+// Elements and wavefronts of a block of a final kernel with nt terms of nch
+// chunks and `outs` outputs per element: one wavefront's lanes full of
+// (element, chunk) pairs when the term values fit in 64 KB of LDS.
+struct FinalShape { int eb, waves; };
+inline FinalShape final_shape(int nt, int nch, int outs, int64_t E) {
+  const int fit = kFinalValues / (nt * outs);
+  if (fit < 1) throw std::runtime_error("final kernel: block too large");
+  int eb = std::max(1, std::min(kWave / std::min(nch, kWave), fit));
+  eb = static_cast<int>(std::min<int64_t>(eb, std::max<int64_t>(E, 1)));
+  return {eb, std::min(nt, 8)};
+}
+
+// Sources requested together: four on small grids, where a launch waits for
+// the longest lists of its few wavefronts, two on large ones, where the
+// registers of four cost more resident wavefronts than the overlap saves
+// (4D sparse grid of 10,496 elements: 9.3 ms a run with two, 8.0 with four;
+// 512 2D instances, 90 to 165 thousand elements: 18.9 and 20.0 ms).
+constexpr int64_t kFewElements = 16384;
+
+template <int PF, int PT, class T>
+void phase_t(const ListTerm* terms, int ntask, int64_t E, int R, const double* u, hipStream_t s) {
+  const dim3 grid(nblocks(E * R), ntask), block(kBlock);
+  const uint32_t e = static_cast<uint32_t>(E), r = static_cast<uint32_t>(R);
+  if (E <= kFewElements) hipLaunchKernelGGL((k_list_phase<PF, PT, T, 4>), grid, block, 0, s, terms, e, r, u);
+  else hipLaunchKernelGGL((k_list_phase<PF, PT, T, 2>), grid, block, 0, s, terms, e, r, u);
+}
+
+template <int PF, int PT, class T>
+void up_final_t(const ListTerm* terms, int nterm, int64_t E, int P, const double* u, T* up, T* fp, const double* vcoef,
+                int kind, double fs, int ncomp, hipStream_t s) {
+  const int R = P / PT;
+  const FinalShape f = final_shape(nterm, R, P, E);
+  const dim3 grid(static_cast<unsigned>((E + f.eb - 1) / f.eb)), block(f.waves * kWave);
+  const size_t lds = sizeof(double) * nterm * f.eb * P;
+  if (E <= kFewElements)
+    hipLaunchKernelGGL((k_list_up_final<PF, PT, T, 4>), grid, block, lds, s, terms, nterm, f.eb, R, E, P, u, up, fp,
+                       vcoef, kind, fs, ncomp);
+  else
+    hipLaunchKernelGGL((k_list_up_final<PF, PT, T, 2>), grid, block, lds, s, terms, nterm, f.eb, R, E, P, u, up, fp,
+                       vcoef, kind, fs, ncomp);
+}
+
+template <int PFM, int PFK, class T>
+void rhs_final_t(const ListTerm* terms, int nterm, int npen, int64_t E, int K, double* rhs, const double* u,
+                 const double* tn, double* u_next, int scheme, int stage, double dt, const double* dtv, int32_t* err,
+                 hipStream_t s) {
+  const int R = K / PFK;
+  const FinalShape f = final_shape(nterm + npen, R, K, E);
+  const dim3 grid(static_cast<unsigned>((E + f.eb - 1) / f.eb)), block(f.waves * kWave);
+  const size_t lds = sizeof(double) * (nterm + npen) * f.eb * K;
+  if (E <= kFewElements)
+    hipLaunchKernelGGL((k_list_rhs_final<PFM, PFK, T, 4>), grid, block, lds, s, terms, nterm, npen, f.eb, R, E, K, rhs,
+                       u, tn, u_next, scheme, stage, dt, dtv, err);
+  else
+    hipLaunchKernelGGL((k_list_rhs_final<PFM, PFK, T, 2>), grid, block, lds, s, terms, nterm, npen, f.eb, R, E, K, rhs,
+                       u, tn, u_next, scheme, stage, dt, dtv, err);
+}
+
+}  // namespace
+
+void list_nonzero(uint8_t* nz, const double* M, int ns, int block, int kind, bool clear, hipStream_t s) {
+  const int64_t n = static_cast<int64_t>(ns) * ns;
+  hipLaunchKernelGGL(k_list_nz, dim3(nblocks(n)), dim3(kBlock), 0, s, nz, M, n, block, 1 << kind, clear ? 1 : 0);
+}
+
+void list_fill_totals(int32_t* total, int n, hipStream_t s) {
+  hipLaunchKernelGGL(k_list_zero, dim3(1), dim3(kWave), 0, s, total, n);
+}
+
+void list_build(const ListBuildArgs& a, int kind0, int nkind, hipStream_t s) {
+  if (a.E > 0)
+    hipLaunchKernelGGL(k_list_build, dim3(nblocks(a.E), nkind * a.D), dim3(kBlock), 0, s, a, kind0);
+}
+
+template <class T>
+void list_phase(int pf1, int pt1, const ListTerm* terms, int ntask, int64_t E, int R, const double* u,
+                hipStream_t s) {
+#define ADG_LP(F, P) if (pf1 == F && pt1 == P) { phase_t<F, P, T>(terms, ntask, E, R, u, s); return; }
+#ifdef ADG_LIST_QUICK
+  ADG_LP(2, 3) ADG_LP(3, 2) ADG_LP(3, 4) ADG_LP(4, 3)
+#else
+  ADG_LP(2, 2) ADG_LP(2, 3) ADG_LP(2, 4) ADG_LP(2, 5) ADG_LP(3, 2) ADG_LP(3, 3) ADG_LP(3, 4) ADG_LP(3, 5)
+  ADG_LP(4, 2) ADG_LP(4, 3) ADG_LP(4, 4) ADG_LP(4, 5) ADG_LP(5, 2) ADG_LP(5, 3) ADG_LP(5, 4)
+#endif
+#undef ADG_LP
+  throw std::runtime_error("list phase: unsupported basis sizes");
+}
+
+template <class T>
+void list_up_final(int k1, int m1, const ListTerm* terms, int nterm, int64_t E, int P, const double* u, T* up,
+                   T* fp, const double* vcoef, int kind, double fs, int ncomp, hipStream_t s) {
+#define ADG_LU(F, Q)                                                                          \
+  if (k1 == F && m1 == Q) {                                                                   \
+    up_final_t<F, Q, T>(terms, nterm, E, P, u, up, fp, vcoef, kind, fs, ncomp, s);        \
+    return;                                                                                   \
+  }
+#ifdef ADG_LIST_QUICK
+  ADG_LU(2, 3) ADG_LU(3, 4)
+#else
+  ADG_LU(2, 2) ADG_LU(2, 3) ADG_LU(2, 4) ADG_LU(2, 5) ADG_LU(3, 2) ADG_LU(3, 3) ADG_LU(3, 4) ADG_LU(3, 5)
+  ADG_LU(4, 2) ADG_LU(4, 3) ADG_LU(4, 4) ADG_LU(4, 5)
+#endif
+#undef ADG_LU
+  throw std::runtime_error("list up final: unsupported basis sizes");
+}
+
+template <class T>
+void list_rhs_final(int m1, int k1, const ListTerm* terms, int nterm, int npen, int64_t E, int K, double* rhs,
+                    const double* u, const double* tn, double* u_next, int scheme, int stage, double dt,
+                    const double* dtv, int32_t* err, hipStream_t s) {
+#define ADG_LR(F, Q)                                                                                               \
+  if (m1 == F && k1 == Q) {                                                                                        \
+    rhs_final_t<F, Q, T>(terms, nterm, npen, E, K, rhs, u, tn, u_next, scheme, stage, dt, dtv, err, s);        \
+    return;                                                                                                        \
+  }
+#ifdef ADG_LIST_QUICK
+  ADG_LR(3, 2) ADG_LR(4, 3)
+#else
+  ADG_LR(2, 2) ADG_LR(2, 3) ADG_LR(2, 4) ADG_LR(3, 2) ADG_LR(3, 3) ADG_LR(3, 4) ADG_LR(4, 2) ADG_LR(4, 3)
+  ADG_LR(4, 4) ADG_LR(5, 2) ADG_LR(5, 3) ADG_LR(5, 4)
+#endif
+#undef ADG_LR
+  throw std::runtime_error("list rhs final: unsupported basis sizes");
+}
+
+#define ADG_LIST_INST(T)                                                                                              \
+  template void list_phase<T>(int, int, const ListTerm*, int, int64_t, int, const double*, hipStream_t);              \
+  template void list_up_final<T>(int, int, const ListTerm*, int, int64_t, int, const double*, T*, T*,            \
+                                 const double*, int, double, int, hipStream_t);                                       \
+  template void list_rhs_final<T>(int, int, const ListTerm*, int, int, int64_t, int, double*, const double*,     \
+                                  const double*, double*, int, int, double, const double*, int32_t*, hipStream_t);
+ADG_LIST_INST(double)
+ADG_LIST_INST(float)
+
+}  // namespace adg

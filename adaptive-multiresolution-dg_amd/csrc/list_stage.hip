@@ -1,0 +1,376 @@
+// Fused RK stage on the source lists (list.hpp): the lists of the current
+// grid, the plan of a stage's sweeps, and the stage itself.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <climits>
+#include <cstring>
+#include <map>
+
+#include "context.hpp"
+#include "list.hpp"
+
+namespace adg {
+
+namespace {
+
+template <class T>
+void upload(DevBuf<T>& b, const std::vector<T>& h, hipStream_t s) {
+  b.ensure(std::max<size_t>(h.size(), 1));
+  if (!h.empty()) hip_check(hipMemcpyAsync(b.p, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice, s), "upload");
+}
+
+int prod_of(const int* sz, int D) {
+  int p = 1;
+  for (int d = 0; d < D; ++d) p *= sz[d];
+  return p;
+}
+
+}  // namespace
+
+// The sweeps of a stage, in launch order, as device descriptors.  They hold
+// buffer addresses but nothing of the grid (its size is a kernel argument and
+// the buffers keep room for more elements), so a plan outlives grid changes.
+struct Context::ListPlan {
+  std::vector<uintptr_t> key;
+  DevBuf<ListTerm> terms;
+  DevBuf<int2> rofs;
+  struct Phase {
+    int first, n, R;
+    double bytes;  // algorithmic bytes per element
+  };
+  std::vector<Phase> up, rhs;
+  Phase up_final, rhs_final;  // rhs_final: the penalty sweeps follow its terms
+};
+
+bool Context::list_stage_fits() const {
+  if (E() == 0) return false;
+  // the kernels use 32-bit work items and byte offsets into the lists, one
+  // component of a sweep's input and the tables, 24-bit products of element
+  // and slot numbers, and count a target's entries in 16 bits
+  const int mx = std::max(k, m) + 1;
+  int64_t T = 1;
+  for (int d = 0; d < D; ++d) T *= mx;
+  const int64_t lim = int64_t{1} << 32, ns = int64_t{1} << nmax;
+  // the last sweeps keep every term value of an element in LDS (all but k = 3
+  // in four dimensions fit: 68 terms of 256 values)
+  const int64_t nord = D == 1 ? 1 : int64_t{1} << (D - 1);
+  if ((2 * D * nord + D) * K > kFinalValues || nord * P > kFinalValues) return false;
+  return E() < (1 << 24) && E() * T * 8 < lim && E() * (4 * nmax + 4) * 8 < lim && ns * ns * mx * mx * 8 < lim;
+}
+
+// Tables whose blocks decide which pairs a list holds.
+void Context::list_nonzero_tables() {
+  const int ns = 1 << nmax, kb = (k + 1) * (m + 1);
+  nz_tab.ensure(static_cast<size_t>(ns) * ns);
+  // (no table: every block counts)
+  list_nonzero(nz_tab.p, nullptr, ns, 1, LIST_VOL, true, stream);
+  list_nonzero(nz_tab.p, t_pt.p, ns, kb, LIST_PT, true, stream);
+  list_nonzero(nz_tab.p, t_la_flx.p, ns, kb, LIST_FLX, true, stream);
+  list_nonzero(nz_tab.p, t_aa[4].p, ns, (k + 1) * (k + 1), LIST_FLX, false, stream);
+  nz_interp = interp;
+}
+
+void Context::ensure_lists(int kind0, int nkind, const uint8_t* nz) {
+  bool ok = true;
+  for (int q = kind0; q < kind0 + nkind; ++q)
+    ok = ok && list_version[q] == grid_version && list_level_cap[q] == lsum_cap && list_interp[q] == interp;
+  if (ok) return;
+  not_recording("source lists");
+  HostTimer timer(*this, HOST_UPLOAD);
+  if (!nz) {
+    if (nz_interp != interp) list_nonzero_tables();
+    nz = nz_tab.p;
+  }
+  ListBuildArgs a{};
+  for (int d = 0; d < D; ++d) {
+    a.slot[d] = g_slot[d].p;
+    a.fbase[d] = g_fbase[d].p;
+    a.fmaxl[d] = g_fmaxl[d].p;
+    a.fmap[d] = g_fmap[d].p;
+    a.fbits[d] = g_fbits[d].p;
+  }
+  a.lsum = g_lsum.p; a.inst = g_inst.p; a.nz = nz; a.err = err_flag.p;
+  a.E = E(); a.D = D; a.ns = 1 << nmax; a.level_cap = lsum_cap;
+  l_total.ensure(LIST_KINDS * kMaxDim);
+  a.total = l_total.p;
+  // An element of level l has at most l + 1 related cells at levels up to its
+  // own in a nested relation, 2 l + 3 in one that counts touching cells, and
+  // as many pairs (less itself) with it as the finer one are in the L parts.
+  for (int d = 0; d < D; ++d) {
+    int lmax = 0;
+    for (int i = 0; i < B(); ++i) lmax = std::max(lmax, inst_lmax[static_cast<size_t>(i) * D + d]);
+    for (int q = kind0; q < kind0 + nkind; ++q) {
+      const bool touch = q == LIST_FLX || q == LIST_LIN;
+      const int64_t room = E() * (touch ? 4 * lmax + 4 : 2 * lmax + 1);
+      const int l = q * D + d;
+      l_meta[l].ensure(static_cast<size_t>(E()));
+      l_ent[l].ensure(static_cast<size_t>(room));
+      a.meta[l] = l_meta[l].p;
+      a.ent[l] = l_ent[l].p;
+      a.cap[l] = static_cast<int64_t>(l_ent[l].cap);
+    }
+  }
+  list_fill_totals(l_total.p + kind0 * D, nkind * D, stream);
+  list_build(a, kind0, nkind, stream);
+  for (int q = kind0; q < kind0 + nkind; ++q) {
+    list_version[q] = grid_version;
+    list_level_cap[q] = lsum_cap;
+    list_interp[q] = interp;
+  }
+}
+
+Context::ListPlan& Context::get_list_plan(const StageProblem& p) {
+  std::vector<std::vector<int>> lus;
+  const std::vector<std::vector<int>> dims = transform_orders(D, lus);
+  const int nord = static_cast<int>(dims.size());
+  if (E() > list_ecap) {
+    not_recording("stage buffers");
+    list_ecap = (E() + E() / 4 + 1023) / 1024 * 1024;
+    list_plan.reset();
+  }
+  u_next.ensure(static_cast<size_t>(E()) * K);
+  auto bits = [](double v) {
+    uintptr_t b;
+    std::memcpy(&b, &v, sizeof b);
+    return b;
+  };
+  auto ptr = [](const void* q) { return reinterpret_cast<uintptr_t>(q); };
+  const double* pen_coef = inst_alpha.empty() ? nullptr : d_pen_coef.p;
+  std::vector<uintptr_t> key = {static_cast<uintptr_t>(same_flux), static_cast<uintptr_t>(is_varcoef(p.flux_kind)),
+                                static_cast<uintptr_t>(interp), static_cast<uintptr_t>(precision), ptr(t_pt.p),
+                                ptr(t_la_uv.p), ptr(t_la_uvx.p), ptr(t_la_flx.p), ptr(fucoe.p), ptr(fucoe32.p),
+                                ptr(list_tmp.p), ptr(pen_coef), pen_coef ? static_cast<uintptr_t>(B()) : 0};
+  for (int d = 0; d < D; ++d) {
+    key.push_back(bits(p.alpha[d]));
+    for (int q = LIST_PT; q <= LIST_FLX; ++q) {
+      key.push_back(ptr(l_meta[q * D + d].p));
+      key.push_back(ptr(l_ent[q * D + d].p));
+    }
+  }
+  if (list_plan && list_plan->key == key) return *list_plan;
+  not_recording("stage plan");
+  HostTimer timer(*this, HOST_PLAN);
+  const bool f32 = precision == 1;
+  const double w = f32 ? 4.0 : 8.0;
+  list_plan.reset(new ListPlan());
+  ListPlan& pl = *list_plan;
+  std::vector<ListTerm> flat;
+  std::vector<int2> rofs;
+  std::map<std::vector<int>, size_t> rofs_at;
+  size_t tmp_used = 0, tmp_most = 0;  // values per element of the phase buffers
+  struct Out { size_t term, at; };
+  std::vector<Out> outs;                        // output buffers, addressed once the size is known
+  std::vector<std::pair<size_t, size_t>> ins;   // inputs that are phase buffers
+  std::vector<size_t> rofs_of;                  // per term: first entry of its offsets
+  auto rest_offsets = [&](const int* sin, const int* sout, int dd) {
+    std::vector<int> id(sin, sin + D);
+    id.insert(id.end(), sout, sout + D);
+    id.push_back(dd);
+    auto it = rofs_at.find(id);
+    if (it != rofs_at.end()) return it->second;
+    const size_t at = rofs.size();
+    rofs_at[id] = at;
+    int R = 1;
+    for (int d = 0; d < D; ++d) R *= d == dd ? 1 : sin[d];
+    for (int r = 0; r < R; ++r) {
+      int rem = r, bi = 0, bo = 0, si = 1, so = 1;
+      for (int d = D - 1; d >= 0; --d) {
+        if (d != dd) {
+          const int q = rem % sin[d];
+          rem /= sin[d];
+          bi += q * si;
+          bo += q * so;
+        }
+        si *= sin[d];
+        so *= sout[d];
+      }
+      rofs.push_back(int2{bi, bo});
+    }
+    return at;
+  };
+  // a term over lists of `kind`; sizes before and after the sweep of dd
+  auto make_term = [&](int kind, const double* in, const float* in32, int comp, const int* sin, const int* sout, int dd,
+                       const double* M, int lu, double coef, bool split) {
+    ListTerm t{};
+    t.in = in; t.in32 = in32; t.M = M; t.ns = 1 << nmax; t.lu = lu; t.coef = coef;
+    if (split) {
+      const SplitTable& sp = split_table(M, (static_cast<size_t>(1) << (2 * nmax)) * sin[dd] * sout[dd]);
+      t.Mh = sp.hi.p;
+      t.Ml = sp.lo.p;
+    }
+    t.meta = l_meta[kind * D + dd].p;
+    t.ent = l_ent[kind * D + dd].p;
+    t.comp = comp;
+    t.comp_size = prod_of(sin, D);
+    t.Tin = prod_of(sin, D);
+    t.Tout = prod_of(sout, D);
+    t.R = t.Tin / sin[dd];
+    t.sdd = t.sod = 1;
+    for (int d = dd + 1; d < D; ++d) { t.sdd *= sin[d]; t.sod *= sout[d]; }
+    rofs_of.push_back(rest_offsets(sin, sout, dd));
+    return t;
+  };
+  auto in_bytes = [&](const ListTerm& t, bool phase_in) { return (phase_in || t.in32 || !f32) ? w : 8.0; };
+  // Chains of partial sums as a prefix tree (one node per distinct leading
+  // sequence of sweeps; Context::fused_plan states why sharing them and
+  // where the coefficient 1/2 is applied leaves every value unchanged).
+  struct Chain {
+    int kind[kMaxDim], comp, o;
+    const double* in;
+    const float* in32;
+    const double* tab[kMaxDim];
+    double coef;
+  };
+  auto build = [&](const std::vector<Chain>& chains, int pf1, int pt1, std::vector<ListPlan::Phase>& phases,
+                   ListPlan::Phase& last) {
+    auto prefix = [&](const Chain& c, int st) {
+      std::vector<uintptr_t> id = {ptr(c.in), static_cast<uintptr_t>(c.comp)};
+      for (int j = 0; j <= st; ++j) {
+        const int dd = dims[c.o][j];
+        id.insert(id.end(), {static_cast<uintptr_t>(dd), ptr(c.tab[dd]), static_cast<uintptr_t>(lus[c.o][j])});
+      }
+      return id;
+    };
+    std::map<std::vector<uintptr_t>, std::vector<double>> coefs;  // coefficients of the chains through a node
+    for (const Chain& c : chains)
+      for (int st = 0; st + 1 < D; ++st) {
+        std::vector<double>& v = coefs[prefix(c, st)];
+        if (std::find(v.begin(), v.end(), c.coef) == v.end()) v.push_back(c.coef);
+      }
+    struct Node { size_t at; bool applied; };  // output of a node; the coefficient is in it
+    std::map<std::vector<uintptr_t>, Node> nodes;
+    tmp_used = 0;
+    phases.clear();
+    for (int st = 0; st < D; ++st) {
+      ListPlan::Phase ph{static_cast<int>(flat.size()), 0, 0, 0.};
+      for (const Chain& c : chains) {
+        const std::vector<uintptr_t> id = prefix(c, st);
+        if (st + 1 < D && nodes.count(id)) continue;
+        int sin[kMaxDim], sout[kMaxDim];
+        for (int d = 0; d < D; ++d) sin[d] = pf1;
+        for (int j = 0; j < st; ++j) sin[dims[c.o][j]] = pt1;
+        std::copy(sin, sin + D, sout);
+        const int dd = dims[c.o][st];
+        sout[dd] = pt1;
+        const Node* before = st ? &nodes.at(prefix(c, st - 1)) : nullptr;
+        const bool applied = before && before->applied;
+        const bool here = !applied && (st + 1 == D || coefs[id].size() == 1);
+        ListTerm t = make_term(c.kind[dd], before ? nullptr : c.in, before ? nullptr : c.in32, before ? 0 : c.comp, sin,
+                               sout, dd, c.tab[dd], lus[c.o][st], here ? c.coef : 1.0, f32);
+        if (before) ins.push_back({flat.size(), before->at});
+        ph.bytes += in_bytes(t, before != nullptr) * t.Tin;
+        if (st + 1 < D) {
+          nodes[id] = {tmp_used, applied || here};
+          outs.push_back({flat.size(), tmp_used});
+          tmp_used += t.Tout;
+          ph.bytes += w * t.Tout;
+        }
+        ph.R = t.R;
+        ++ph.n;
+        flat.push_back(t);
+      }
+      if (st + 1 < D) phases.push_back(ph);
+      else last = ph;
+    }
+    tmp_most = std::max(tmp_most, tmp_used);
+  };
+  std::vector<Chain> chains;
+  for (int o = 0; o < nord; ++o) {
+    Chain c{};
+    c.o = o;
+    c.coef = 1.0;
+    for (int d = 0; d < D; ++d) { c.kind[d] = LIST_PT; c.tab[d] = t_pt.p; }
+    chains.push_back(c);
+  }
+  build(chains, k + 1, m + 1, pl.up, pl.up_final);
+  const int nc = same_flux ? 1 : D;
+  pl.up_final.bytes += w * P * (1 + nc) + (is_varcoef(p.flux_kind) ? 8.0 * P * nc : 0.);
+  chains.clear();
+  // in the reference order: volume terms for d = 0..D-1, then flux terms
+  for (int ft = 0; ft < 2; ++ft)
+    for (int d = 0; d < D; ++d)
+      for (int o = 0; o < nord; ++o) {
+        Chain c{};
+        c.o = o;
+        c.comp = same_flux ? 0 : d;
+        c.in = fucoe.p;
+        c.in32 = f32 ? fucoe32.p : nullptr;
+        c.coef = ft ? 0.5 : 1.0;
+        for (int dd = 0; dd < D; ++dd) {
+          c.kind[dd] = dd == d && ft ? LIST_FLX : LIST_VOL;
+          c.tab[dd] = dd == d ? (ft ? t_la_flx.p : t_la_uvx.p) : t_la_uv.p;
+        }
+        chains.push_back(c);
+      }
+  build(chains, m + 1, k + 1, pl.rhs, pl.rhs_final);
+  pl.rhs_final.bytes += 8.0 * K * (1 + 3 + D);
+  // the LF penalty stays FP64 in every precision
+  int ksz[kMaxDim];
+  for (int d = 0; d < D; ++d) ksz[d] = k + 1;
+  for (int d = 0; d < D; ++d) {
+    flat.push_back(make_term(LIST_FLX, nullptr, nullptr, 0, ksz, ksz, d, t_aa[4].p, LU_FULL, -p.alpha[d] / 2., false));
+    if (pen_coef) flat.back().coef_inst = pen_coef + static_cast<size_t>(d) * B();
+  }
+  list_tmp.ensure(std::max<size_t>(tmp_most * list_ecap, 1));
+  key[10] = ptr(list_tmp.p);
+  upload(pl.rofs, rofs, stream);
+  for (const Out& o : outs) flat[o.term].out = list_tmp.p + o.at * list_ecap;
+  for (const auto& i : ins) {
+    flat[i.first].in = list_tmp.p + i.second * list_ecap;
+    if (f32) flat[i.first].in32 = reinterpret_cast<const float*>(flat[i.first].in);
+  }
+  for (size_t i = 0; i < flat.size(); ++i) flat[i].rofs = pl.rofs.p + rofs_of[i];
+  upload(pl.terms, flat, stream);
+  sync();  // the host vectors are gone after this call
+  pl.key = key;
+  return pl;
+}
+
+template <class T>
+void Context::stage_list(const StageProblem& p, int scheme, int stage, double dt) {
+  ensure_lists(LIST_PT, 3, nullptr);
+  ListPlan& pl = get_list_plan(p);
+  constexpr bool f32 = sizeof(T) == 4;
+  const int up_kind = interp == 1 ? -1 : p.flux_kind;
+  const int ncomp = same_flux ? 1 : D;
+  T* upp;
+  T* fpp;
+  if constexpr (f32) { upp = up32.p; fpp = fp32.p; }
+  else { upp = up.p; fpp = fp.p; }
+  const int64_t n = E();
+  auto phases = [&](const std::vector<ListPlan::Phase>& phs, int cat, int pf1, int pt1) {
+    for (const ListPlan::Phase& ph : phs) {
+      prof_begin(cat, ph.bytes * n);
+      list_phase<T>(pf1, pt1, pl.terms.p + ph.first, ph.n, n, ph.R, u.p, stream);
+      ++stage_launches;
+      prof_end();
+    }
+  };
+  phases(pl.up, PROF_SWEEP, k + 1, m + 1);
+  prof_begin(PROF_FLUX, pl.up_final.bytes * n);
+  list_up_final<T>(k + 1, m + 1, pl.terms.p + pl.up_final.first, pl.up_final.n, n, P, u.p, upp, fpp, vcoef.p,
+                   up_kind, p.flux_param, ncomp, stream);
+  ++stage_launches;
+  if (interp == 1) {
+    flux_herm<T>(upp, fpp, p.flux_kind, T(p.flux_param), ncomp);
+    ++stage_launches;
+  }
+  prof_end();
+  if constexpr (f32) surplus_transform32(fp32.p, fucoe32.p, interA32.p, interB32.p, ncomp);
+  else surplus_transform(fp.p, fucoe.p, interA.p, interB.p, ncomp);
+  stage_launches += D;
+  phases(pl.rhs, PROF_RHS_PHASE, m + 1, k + 1);
+  prof_begin(PROF_RK, pl.rhs_final.bytes * n);
+  list_rhs_final<T>(m + 1, k + 1, pl.terms.p + pl.rhs_final.first, pl.rhs_final.n, D, n, K, rhs.p, u.p, tn.p,
+                    u_next.p, scheme, stage, dt, use_inst_dt ? d_inst_dt.p : nullptr, err_flag.p, stream);
+  ++stage_launches;
+  prof_end();
+  std::swap(u.p, u_next.p);
+  std::swap(u.cap, u_next.cap);
+}
+
+template void Context::stage_list<double>(const StageProblem&, int, int, double);
+template void Context::stage_list<float>(const StageProblem&, int, int, double);
+
+}  // namespace adg

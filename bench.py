@@ -214,9 +214,8 @@ def main():
                     help="chosen form: thread mapping of every fused kernel (-1: the autotuner picks per class)")
     ap.add_argument("--mappings", default=None,
                     help="chosen form: thread mapping per fused kernel class (eval-up phases, eval-up final, "
-                         "right-hand-side phases, right-hand-side final), e.g. 3,3,7,7, or 'auto' for the "
-                         "autotuner; default 3,3,7,7 on c4 (the best per class in a sweep of all ten mappings "
-                         "at the per-context size), auto elsewhere")
+                         "right-hand-side phases, right-hand-side final), e.g. 3,3,7,7; default 'auto': the "
+                         "sweeps over source lists")
     ap.add_argument("--graph", type=int, default=0, choices=(0, 1),
                     help="chosen form: record whole RK steps into HIP graphs and replay them (adg_set_graph_step)")
     ap.add_argument("--adapt", default="device", choices=("host", "device"),
@@ -269,7 +268,7 @@ def main():
                 bsols.append(b)
     prec = pyadg.PREC_FP32_SPLIT if args.precision == "fp32" else pyadg.PREC_FP64
     if args.mappings is None:
-        args.mappings = "3,3,7,7" if args.workload == "c4" else "auto"
+        args.mappings = "auto"
     mappings = [] if args.mappings == "auto" else [int(v) for v in args.mappings.split(",")]
     if mappings and prec == pyadg.PREC_FP32_SPLIT:  # classes 4..7 are the FP32 ones
         mappings = [-1] * 4 + mappings
@@ -445,7 +444,10 @@ def main():
             for (kc, bucket), v in c.kernel_tuning().items():
                 if kc == cls:
                     tuning[bucket] = v
-        if cat in ("sweep", "rhs_phase") and len(set(tuning.values())) == 1:
+        if fixed < 0 and not tuning:  # no class fixed: the stage on source lists
+            kernel = {"sweep": "k_list_phase (eval-up)", "rhs_phase": "k_list_phase (right-hand side)",
+                      "flux": "k_list_up_final", "rk": "k_list_rhs_final"}[cat]
+        elif cat in ("sweep", "rhs_phase") and len(set(tuning.values())) == 1:
             v = next(iter(tuning.values()))
             pf, pt = (w.k + 1, w.m + 1) if cat == "sweep" else (w.m + 1, w.k + 1)
             ty = "float" if prec == pyadg.PREC_FP32_SPLIT else "double"

@@ -1,0 +1,72 @@
+"""The stage on source lists (the form that runs when no mapping is fixed)
+against the fused per-element kernels and the per-sweep path, bit for bit:
+every basis size the fused stage provides, both interpolation families, the
+level-sum cap, FP32 storage, and grids on both sides of the size at which the
+kernels request more sources at a time (16,384 elements)."""
+import numpy as np
+import pytest
+
+import pyadg
+import workloads
+from common import first_diff, ic_params, problem
+
+pytestmark = pytest.mark.gpu
+
+
+def _steps(s, prob, variant, steps, form=1):
+    s.set_kernel_variant(variant)
+    s.restore_state(0)
+    p = pyadg.Problem.from_buffer_copy(prob)
+    p.form, p.max_steps, p.t_start = form, steps, 0.0
+    s.run_hyperbolic(p)
+    return s.num_elem, s.get()
+
+
+def _same(a, b, what):
+    assert a[0] == b[0], f"{what}: {a[0]} and {b[0]} elements"
+    assert np.array_equal(a[1], b[1]), f"{what}: " + first_diff(a[1], b[1])
+
+
+@pytest.mark.parametrize("dim,k,m,nmax", [(1, 2, 3, 7), (1, 1, 1, 1), (2, 1, 4, 5), (2, 2, 1, 4), (2, 3, 2, 4),
+                                          (3, 1, 1, 3), (3, 2, 2, 3), (3, 3, 4, 3), (4, 1, 3, 3), (4, 2, 3, 2),
+                                          (4, 3, 4, 1)])
+def test_basis_sizes(dim, k, m, nmax):
+    print(f"[case] lists dim={dim} k={k} m={m} nmax={nmax}", flush=True)
+    s = pyadg.Solution(dim, k, m, nmax, True, nmax)
+    s.init_adaptive_intp_builtin(ic_params(1, shift=0.13), 1e10)
+    s.save_state(0)
+    for flux in (pyadg.FLUX_BURGERS, pyadg.FLUX_VARCOEF):
+        p = problem(flux_kind=flux, flux_param=0.4, alpha=[1.3] * dim, wave_speed=[1.0] * dim, cfl=0.05, t_final=1.0,
+                    adaptive=0, eps=0.0, eta=0.0, max_steps=0, t_start=0.0)
+        got = _steps(s, p, -1, 2)
+        _same(got, _steps(s, p, 1, 2), f"flux {flux}, per-element kernels")
+        _same(got, _steps(s, p, -1, 2, form=0), f"flux {flux}, per-sweep path")
+
+
+@pytest.mark.parametrize("herm,fp32,cap", [(1, 0, -1), (0, 1, -1), (0, 0, 3), (1, 1, 4)])
+def test_family_precision_cap(herm, fp32, cap):
+    print(f"[case] lists herm={herm} fp32={fp32} cap={cap}", flush=True)
+    ws = [workloads.c2_burgers(seed=i, nmax=6, level_init=5) for i in (3, 4, 5)]
+    s = workloads.make_batch(ws)
+    s.set_interpolation(herm)
+    s.set_precision(fp32)
+    s.set_level_sum_cap(cap)
+    s.save_state(0)
+    _same(_steps(s, ws[0].problem, -1, 3), _steps(s, ws[0].problem, 3, 3), "per-element kernels")
+    # the other family on the same grid rebuilds the lists of its tables
+    s.set_interpolation(1 - herm)
+    _same(_steps(s, ws[0].problem, -1, 1), _steps(s, ws[0].problem, 3, 1), "other family")
+
+
+@pytest.mark.parametrize("batch", [60, 110])
+def test_few_and_many_elements(batch):
+    print(f"[case] lists batch={batch}", flush=True)
+    ws = [workloads.c2_burgers(seed=i + 1, nmax=6, level_init=5) for i in range(batch)]
+    s = workloads.make_batch(ws)
+    assert (s.num_elem > 16384) == (batch == 110), s.num_elem
+    s.save_state(0)
+    p = pyadg.Problem.from_buffer_copy(ws[0].problem)
+    p.adaptive = 0
+    _same(_steps(s, p, -1, 1), _steps(s, p, 3, 1), "fixed grid")
+    # refinement and coarsening grow and shrink the lists
+    _same(_steps(s, ws[0].problem, -1, 2), _steps(s, ws[0].problem, 3, 2), "adaptive")
