@@ -535,7 +535,7 @@ int adg_set_interpolation(adg_ctx* h, int family) {
 int adg_set_level_sum_cap(adg_ctx* h, int cap) {
   return guard(h, [&](adg::Context& c) { c.lsum_cap = cap < 0 ? -1 : cap; });
 }
-int adg_eval_up(adg_ctx* h) { return guard(h, [](adg::Context& c) { c.eval_up(); }, kDeviceTables); }
+int adg_eval_up(adg_ctx* h) { return guard(h, [](adg::Context& c) { c.eval_up_op(); }, kDeviceTables); }
 int adg_flux(adg_ctx* h, int kind, const double* params) {
   return guard(h, [&](adg::Context& c) {
     if (kind < 0 || kind > 2) throw std::runtime_error("unknown flux kind");
@@ -558,10 +558,10 @@ int adg_fp_to_coe(adg_ctx* h) {
   }, kDeviceTables);
 }
 int adg_rhs_zero(adg_ctx* h) { return guard(h, [](adg::Context& c) { c.rhs_zero(); }, kDeviceTables); }
-int adg_rhs_lagr_vol(adg_ctx* h) { return guard(h, [](adg::Context& c) { c.rhs_lagr(false); }, kDeviceTables); }
-int adg_rhs_lagr_flx(adg_ctx* h) { return guard(h, [](adg::Context& c) { c.rhs_lagr(true); }, kDeviceTables); }
-int adg_rhs_penalty(adg_ctx* h, const double* alpha) { return guard(h, [&](adg::Context& c) { c.rhs_penalty(alpha); }, kDeviceTables); }
-int adg_rhs_linear(adg_ctx* h, const double* coef) { return guard(h, [&](adg::Context& c) { c.rhs_linear(coef); }); }
+int adg_rhs_lagr_vol(adg_ctx* h) { return guard(h, [](adg::Context& c) { c.rhs_lagr_op(false); }, kDeviceTables); }
+int adg_rhs_lagr_flx(adg_ctx* h) { return guard(h, [](adg::Context& c) { c.rhs_lagr_op(true); }, kDeviceTables); }
+int adg_rhs_penalty(adg_ctx* h, const double* alpha) { return guard(h, [&](adg::Context& c) { c.rhs_penalty_op(alpha); }, kDeviceTables); }
+int adg_rhs_linear(adg_ctx* h, const double* coef) { return guard(h, [&](adg::Context& c) { c.rhs_linear_op(coef); }); }
 int adg_rk_init(adg_ctx* h) { return guard(h, [](adg::Context& c) { c.rk_init(); }, kDeviceTables); }
 int adg_rk_stage(adg_ctx* h, int scheme, int stage, double dt) {
   return guard(h, [&](adg::Context& c) {
@@ -766,12 +766,7 @@ int adg_run_linear(adg_ctx* h, const double* coef, double dt, int64_t nsteps, ad
     c.sync();
     const auto t0 = std::chrono::steady_clock::now();
     for (int64_t n = 0; n < nsteps; ++n) {
-      c.rk_init();
-      for (int s = 0; s < 3; ++s) {
-        c.rhs_zero();
-        c.rhs_linear(coef);
-        c.rk_stage(ADG_RK3, s, dt);
-      }
+      for (int s = 0; s < 3; ++s) c.linear_stage(coef, ADG_RK3, s, dt, s == 0);
     }
     c.sync();
     c.check_error_flag();

@@ -18,6 +18,7 @@
 namespace adg {
 
 struct TaskDev;
+struct ListRhs;
 
 struct HipError : std::runtime_error {
   using std::runtime_error::runtime_error;
@@ -294,19 +295,38 @@ class Context {
     double flux_param = 0.;
     double alpha[kMaxDim] = {0, 0, 0, 0};
   };
-  void stage_fused(const StageProblem& p, int scheme, int stage, double dt);
+  // first: u^n <- u before the stage
+  void stage_fused(const StageProblem& p, int scheme, int stage, double dt, bool first = false);
   struct FusedPlan;
   FusedPlan& fused_plan(const StageProblem& p);
   template <class T>
   void stage_body(const StageProblem& p, FusedPlan& pl, int scheme, int stage, double dt);
   // The stage on source lists (list.hpp), the form that runs unless the caller
   // fixed a mapping for one of its kernel classes: list_stage.hip.
+  enum ListForm { LIST_STAGE = 0, LIST_OPS, LIST_LINEAR, LIST_FORMS };
+  struct ListPhase;
   struct ListPlan;
-  std::shared_ptr<ListPlan> list_plan;
+  std::shared_ptr<ListPlan> list_plans[LIST_FORMS];
   bool list_stage_fits() const;
-  ListPlan& get_list_plan(const StageProblem& p);
+  ListPlan& get_list_plan(ListForm form);
   template <class T>
-  void stage_list(const StageProblem& p, int scheme, int stage, double dt);
+  void list_phases(const ListPlan& pl, const std::vector<ListPhase>& phases, int cat, int pf1, int pt1);
+  // alpha: LF constants of the penalty terms (null: their coefficients are 1)
+  ListRhs list_rhs(bool add, int scheme, int stage, double dt, bool first, const double* alpha) const;
+  // first: the stage is a step's first (u^n <- u before it)
+  template <class T>
+  void stage_list(const StageProblem& p, int scheme, int stage, double dt, bool first);
+  // eval_up, rhs_lagr, rhs_penalty and rhs_linear on lists where they fit
+  // (the single operators of the C-ABI; the plain form keeps one launch per sweep)
+  bool list_ops_fit() const;
+  void eval_up_op();
+  void rhs_lagr_op(bool flux_term);
+  void rhs_penalty_op(const double* alpha);
+  void rhs_linear_op(const double* coef);
+  void linear_stage(const double* coef, int scheme, int stage, double dt, bool first);
+  void linear_list(const double* coef, bool run, int scheme, int stage, double dt, bool first);
+  void linear_tables(const double* coef);  // t_lin and nz_lin for these speeds
+  DevBuf<uint8_t> nz_lin;
   template <class T>
   void flux_herm(const T* up, T* fp, int kind, T s, int ncomp);
   // lists of the given kinds for the current grid, level-sum cap and

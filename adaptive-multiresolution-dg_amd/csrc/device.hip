@@ -1116,12 +1116,35 @@ void Context::upload_inst_alpha() {
   upload(d_pen_coef, pc, stream);
 }
 
-void Context::rhs_linear(const double* coef) {
-  if (lin_coef.size() != static_cast<size_t>(D) || !std::equal(lin_coef.begin(), lin_coef.end(), coef)) {
-    OperatorTables aa(alpt, alpt);
-    for (int d = 0; d < D; ++d) upload(t_lin[d], to_blocks(linear_operator_table(aa, coef[d]), 1 << nmax, k + 1, k + 1), stream);
-    lin_coef.assign(coef, coef + D);
+// Constant-coefficient operator tables (linear_operator_table of setup.cpp,
+// formed from the tables on the device with the same products and sums).
+__global__ __launch_bounds__(kBlock) void k_linear_table(const double* uvx, const double* flx, double coef, double* out,
+                                                         int64_t n) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  double a = coef * uvx[i], b = coef * flx[i];
+  if (!(fabs(a) >= ROUND_OFF)) a = 0.;
+  if (!(fabs(b) >= ROUND_OFF)) b = 0.;
+  out[i] = a + b;
+}
+
+void Context::linear_tables(const double* coef) {
+  if (lin_coef.size() == static_cast<size_t>(D) && std::equal(lin_coef.begin(), lin_coef.end(), coef)) return;
+  const int ns = 1 << nmax, kb = (k + 1) * (k + 1);
+  const int64_t n = static_cast<int64_t>(ns) * ns * kb;
+  nz_lin.ensure(static_cast<size_t>(ns) * ns);
+  for (int d = 0; d < D; ++d) {
+    t_lin[d].ensure(static_cast<size_t>(n));
+    hipLaunchKernelGGL(k_linear_table, dim3(nblocks(n)), dim3(kBlock), 0, stream, t_aa[1].p,
+                       coef[d] >= 0 ? t_aa[2].p : t_aa[3].p, coef[d], t_lin[d].p, n);
+    list_nonzero(nz_lin.p, t_lin[d].p, ns, kb, LIST_LIN, d == 0, stream);
   }
+  lin_coef.assign(coef, coef + D);
+  list_version[LIST_LIN] = -1;
+}
+
+void Context::rhs_linear(const double* coef) {
+  linear_tables(coef);
   for (int d = 0; d < D; ++d) rhs_single_dim({t_lin[d].p, 1 << nmax}, d, 1.0);
 }
 
@@ -1482,7 +1505,7 @@ void Context::tile_launch(int v, int pf1, int pt1, const TaskDev* tasks, int R, 
   tile_sweep<T>(pf1, pt1, tasks, ntask, ts.ntile, ts.max_tile, tb, te, D, lsum_cap, allr, last, stream);
 }
 
-void Context::stage_fused(const StageProblem& p, int scheme, int stage, double dt) {
+void Context::stage_fused(const StageProblem& p, int scheme, int stage, double dt, bool first) {
   if (E() == 0) return;
   if (is_varcoef(p.flux_kind) &&
       (flux_kind != p.flux_kind || flux_param != p.flux_param || vcoef_version != grid_version)) {
@@ -1505,10 +1528,11 @@ void Context::stage_fused(const StageProblem& p, int scheme, int stage, double d
   for (int c = 0; c < 4; ++c) fixed = fixed || class_variant[c + (precision == 1 ? 4 : 0)] >= 0;
   if (!fixed && list_stage_fits()) {
     ++stage_count;
-    if (precision == 1) stage_list<float>(p, scheme, stage, dt);
-    else stage_list<double>(p, scheme, stage, dt);
+    if (precision == 1) stage_list<float>(p, scheme, stage, dt, first);
+    else stage_list<double>(p, scheme, stage, dt, first);
     return;
   }
+  if (first) rk_init();
   FusedPlan& pl = fused_plan(p);
   ++stage_count;
   if (precision == 1) stage_body<float>(p, pl, scheme, stage, dt);
@@ -1698,8 +1722,7 @@ void Context::not_recording(const char* what) const {
 }
 
 void Context::rk_step_eager(const StageProblem& p, int scheme, int nstage, double dt) {
-  rk_init();
-  for (int s = 0; s < nstage; ++s) stage_fused(p, scheme, s, dt);
+  for (int s = 0; s < nstage; ++s) stage_fused(p, scheme, s, dt, s == 0);
 }
 
 // Everything a recorded step depends on besides the contents of device
@@ -1728,7 +1751,7 @@ std::vector<uintptr_t> Context::step_key(const StageProblem& p, int scheme, int 
       static_cast<uintptr_t>(use_inst_dt), use_inst_dt ? ptr(d_inst_dt.p) : bits(dt), inst_alpha.size()};
   for (int d = 0; d < D; ++d) key.push_back(bits(p.alpha[d]));
   for (int64_t v : list_version) key.push_back(static_cast<uintptr_t>(v));
-  key.insert(key.end(), {ptr(list_plan.get()), ptr(list_tmp.p)});
+  key.insert(key.end(), {ptr(list_plans[LIST_STAGE].get()), ptr(list_tmp.p)});
   if (key[kKeyU] != ptr(u.p) || key[kKeyUNext] != ptr(u_next.p)) throw std::logic_error("step key layout");
   return key;
 }

@@ -75,9 +75,23 @@ template <class T>
 void list_phase(int pf1, int pt1, const ListTerm* terms, int ntask, int64_t E, int R, const double* u, hipStream_t s);
 template <class T>
 void list_up_final(int k1, int m1, const ListTerm* terms, int nterm, int64_t E, int P, const double* u, T* up, T* fp, const double* vcoef, int kind, double fs, int ncomp, hipStream_t s);
+// What the last sweeps of a right-hand side end in.
+struct ListRhs {
+  double* rhs;
+  int add;            // 1: the terms are added to rhs, 0: it is replaced
+  const double* u;    // current coefficients
+  double* u_next;     // RK stage update (null: the right-hand side alone)
+  const double* tn;   // u^n
+  double* tn_store;   // null, or where a step's first stage keeps u^n (tn is u then)
+  int scheme, stage;
+  double dt;
+  const double* dtv;  // per-instance step sizes (null: dt)
+  int32_t* err;
+  double coef[kMaxDimK];  // coefficients of the npen last terms (their own are not read)
+};
+// nterm terms of m1 x k1 blocks, then npen of k1 x k1 blocks on the coefficients
 template <class T>
-void list_rhs_final(int m1, int k1, const ListTerm* terms, int nterm, int npen, int64_t E, int K, double* rhs,
-                    const double* u, const double* tn, double* u_next, int scheme, int stage, double dt,
-                    const double* dtv, int32_t* err, hipStream_t s);
+void list_rhs_final(int m1, int k1, const ListTerm* terms, int nterm, int npen, int64_t E, int K, const ListRhs& r,
+                    hipStream_t s);
 
 }  // namespace adg

@@ -230,12 +230,13 @@ __device__ __forceinline__ void list_sum(const ListTerm& t, const ListIn<T, PF>&
 
 // Term t for rest index c of element e, to out (the element's values).
 template <int PF, int PT, class T, int NB, class O>
-__device__ __forceinline__ void list_item(const ListTerm& t, const ListIn<T, PF>& src, uint32_t e, uint32_t c, O* out) {
+__device__ __forceinline__ void list_item(const ListTerm& t, const ListIn<T, PF>& src, uint32_t e, uint32_t c,
+                                          double coef, O* out) {
   const vi4 meta = gl<vi4>(t.meta, e * 16);
   const vi2 o = gl<vi2>(t.rofs, c * 8);
   T acc[PT];
   list_sum<PF, PT, T, NB>(t, src, meta, o.x, acc);
-  const T cf = T(t.coef_inst ? gl<double>(t.coef_inst, meta.w * 8) : t.coef);
+  const T cf = T(t.coef_inst ? gl<double>(t.coef_inst, meta.w * 8) : coef);
   const int sod = t.sod;
 #pragma unroll
   for (int i = 0; i < PT; ++i) out[o.y + i * sod] = O(acc[i] * cf);
@@ -250,7 +251,7 @@ __global__ __launch_bounds__(kBlock) void k_list_phase(const ListTerm* terms, ui
   const uint32_t e = i / R, c = i - e * R;
   if (e >= E) return;
   const ListIn<T, PF> src(t, u, E);
-  list_item<PF, PT, T, NB>(t, src, e, c, static_cast<T*>(t.out) + static_cast<int64_t>(e) * t.Tout);
+  list_item<PF, PT, T, NB>(t, src, e, c, t.coef, static_cast<T*>(t.out) + static_cast<int64_t>(e) * t.Tout);
 }
 
 // Last sweep of every eval_up partial sum, added in order into the point
@@ -269,7 +270,8 @@ __global__ __launch_bounds__(512) void k_list_up_final(const ListTerm* terms, in
     const ListIn<T, PF> src(terms[t], u, E);
     for (int it = lane; it < ne * nch; it += kWave) {
       const int el = it / nch, c = it - el * nch;
-      list_item<PF, PT, T, NB>(terms[t], src, static_cast<uint32_t>(e0) + el, c, vals + (t * EB + el) * P);
+      list_item<PF, PT, T, NB>(terms[t], src, static_cast<uint32_t>(e0) + el, c,
+                                  terms[t].coef, vals + (t * EB + el) * P);
     }
   }
   __syncthreads();
@@ -288,9 +290,7 @@ __global__ __launch_bounds__(512) void k_list_up_final(const ListTerm* terms, in
 // added in order, then the RK stage update.  Blocks as above.
 template <int PFM, int PFK, class T, int NB>
 __global__ __launch_bounds__(512) void k_list_rhs_final(const ListTerm* terms, int nterm, int npen, int EB, int nch,
-                                                         int64_t E, int K, double* rhs, const double* u,
-                                                         const double* tn, double* u_next, int scheme, int stage,
-                                                         double dt, const double* dtv, int32_t* err) {
+                                                        int64_t E, int K, ListRhs a) {
   extern __shared__ double vals[];  // [nterm + npen][EB][K]
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), W = blockDim.x / kWave;
   const int lane = threadIdx.x % kWave;
@@ -301,22 +301,27 @@ __global__ __launch_bounds__(512) void k_list_rhs_final(const ListTerm* terms, i
       const int el = it / nch, c = it - el * nch;
       double* out = vals + (t * EB + el) * K;
       if (t < nterm)
-        list_item<PFM, PFK, T, NB>(terms[t], ListIn<T, PFM>(terms[t], u, E), static_cast<uint32_t>(e0) + el, c, out);
+        list_item<PFM, PFK, T, NB>(terms[t], ListIn<T, PFM>(terms[t], a.u, E), static_cast<uint32_t>(e0) + el, c,
+                                    terms[t].coef, out);
       else
-        list_item<PFK, PFK, double, NB>(terms[t], ListIn<double, PFK>(terms[t], u, E), static_cast<uint32_t>(e0) + el, c, out);
+        list_item<PFK, PFK, double, NB>(terms[t], ListIn<double, PFK>(terms[t], a.u, E), static_cast<uint32_t>(e0) + el,
+                                        c, a.coef[t - nterm], out);
     }
   }
   __syncthreads();
   const int4* meta = terms[0].meta;
   for (int o = threadIdx.x; o < ne * K; o += blockDim.x) {
-    double r = 0.;
-    for (int j = 0; j < nterm + npen; ++j) r += vals[j * EB * K + o];
     const int64_t gid = e0 * K + o;
-    rhs[gid] = r;
-    const double dte = dtv ? dtv[meta[e0 + o / K].w] : dt;
-    const double un = rk_combine(scheme, stage, dte, tn[gid], u[gid], r);
-    u_next[gid] = un;
-    if (!isfinite(un)) atomicOr(err, ERR_NONFINITE);
+    double r = a.add ? a.rhs[gid] : 0.;
+    for (int j = 0; j < nterm + npen; ++j) r += vals[j * EB * K + o];
+    a.rhs[gid] = r;
+    if (!a.u_next) continue;
+    const double dte = a.dtv ? a.dtv[meta[e0 + o / K].w] : a.dt;
+    const double t = a.tn[gid];
+    if (a.tn_store) a.tn_store[gid] = t;
+    const double un = rk_combine(a.scheme, a.stage, dte, t, a.u[gid], r);
+    a.u_next[gid] = un;
+    if (!isfinite(un)) atomicOr(a.err, ERR_NONFINITE);
   }
 }
 
@@ -363,19 +368,15 @@ void up_final_t(const ListTerm* terms, int nterm, int64_t E, int P, const double
 }
 
 template <int PFM, int PFK, class T>
-void rhs_final_t(const ListTerm* terms, int nterm, int npen, int64_t E, int K, double* rhs, const double* u,
-                 const double* tn, double* u_next, int scheme, int stage, double dt, const double* dtv, int32_t* err,
-                 hipStream_t s) {
+void rhs_final_t(const ListTerm* terms, int nterm, int npen, int64_t E, int K, const ListRhs& r, hipStream_t s) {
   const int R = K / PFK;
   const FinalShape f = final_shape(nterm + npen, R, K, E);
   const dim3 grid(static_cast<unsigned>((E + f.eb - 1) / f.eb)), block(f.waves * kWave);
   const size_t lds = sizeof(double) * (nterm + npen) * f.eb * K;
   if (E <= kFewElements)
-    hipLaunchKernelGGL((k_list_rhs_final<PFM, PFK, T, 4>), grid, block, lds, s, terms, nterm, npen, f.eb, R, E, K, rhs,
-                       u, tn, u_next, scheme, stage, dt, dtv, err);
+    hipLaunchKernelGGL((k_list_rhs_final<PFM, PFK, T, 4>), grid, block, lds, s, terms, nterm, npen, f.eb, R, E, K, r);
   else
-    hipLaunchKernelGGL((k_list_rhs_final<PFM, PFK, T, 2>), grid, block, lds, s, terms, nterm, npen, f.eb, R, E, K, rhs,
-                       u, tn, u_next, scheme, stage, dt, dtv, err);
+    hipLaunchKernelGGL((k_list_rhs_final<PFM, PFK, T, 2>), grid, block, lds, s, terms, nterm, npen, f.eb, R, E, K, r);
 }
 
 }  // namespace
@@ -427,13 +428,12 @@ void list_up_final(int k1, int m1, const ListTerm* terms, int nterm, int64_t E, 
 }
 
 template <class T>
-void list_rhs_final(int m1, int k1, const ListTerm* terms, int nterm, int npen, int64_t E, int K, double* rhs,
-                    const double* u, const double* tn, double* u_next, int scheme, int stage, double dt,
-                    const double* dtv, int32_t* err, hipStream_t s) {
-#define ADG_LR(F, Q)                                                                                               \
-  if (m1 == F && k1 == Q) {                                                                                        \
-    rhs_final_t<F, Q, T>(terms, nterm, npen, E, K, rhs, u, tn, u_next, scheme, stage, dt, dtv, err, s);        \
-    return;                                                                                                        \
+void list_rhs_final(int m1, int k1, const ListTerm* terms, int nterm, int npen, int64_t E, int K, const ListRhs& r,
+                    hipStream_t s) {
+#define ADG_LR(F, Q)                                                \
+  if (m1 == F && k1 == Q) {                                         \
+    rhs_final_t<F, Q, T>(terms, nterm, npen, E, K, r, s);           \
+    return;                                                         \
   }
 #ifdef ADG_LIST_QUICK
   ADG_LR(3, 2) ADG_LR(4, 3)
@@ -449,8 +449,7 @@ void list_rhs_final(int m1, int k1, const ListTerm* terms, int nterm, int npen, 
   template void list_phase<T>(int, int, const ListTerm*, int, int64_t, int, const double*, hipStream_t);              \
   template void list_up_final<T>(int, int, const ListTerm*, int, int64_t, int, const double*, T*, T*,            \
                                  const double*, int, double, int, hipStream_t);                                       \
-  template void list_rhs_final<T>(int, int, const ListTerm*, int, int, int64_t, int, double*, const double*,     \
-                                  const double*, double*, int, int, double, const double*, int32_t*, hipStream_t);
+  template void list_rhs_final<T>(int, int, const ListTerm*, int, int, int64_t, int, const ListRhs&, hipStream_t);
 ADG_LIST_INST(double)
 ADG_LIST_INST(float)
 

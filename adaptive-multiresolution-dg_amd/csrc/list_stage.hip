@@ -4,7 +4,6 @@
 
 #include <algorithm>
 #include <climits>
-#include <cstring>
 #include <map>
 
 #include "context.hpp"
@@ -31,16 +30,18 @@ int prod_of(const int* sz, int D) {
 // The sweeps of a stage, in launch order, as device descriptors.  They hold
 // buffer addresses but nothing of the grid (its size is a kernel argument and
 // the buffers keep room for more elements), so a plan outlives grid changes.
+struct Context::ListPhase {
+  int first = 0, n = 0, R = 0;
+  double bytes = 0.;  // algorithmic bytes per element
+};
 struct Context::ListPlan {
   std::vector<uintptr_t> key;
   DevBuf<ListTerm> terms;
   DevBuf<int2> rofs;
-  struct Phase {
-    int first, n, R;
-    double bytes;  // algorithmic bytes per element
-  };
-  std::vector<Phase> up, rhs;
-  Phase up_final, rhs_final;  // rhs_final: the penalty sweeps follow its terms
+  using Phase = ListPhase;
+  std::vector<Phase> up, rhs, flx;
+  Phase up_final, rhs_final, flx_final;
+  int pen = 0;  // the D penalty sweeps (after rhs_final's terms in the stage's plan)
 };
 
 bool Context::list_stage_fits() const {
@@ -120,38 +121,36 @@ void Context::ensure_lists(int kind0, int nkind, const uint8_t* nz) {
   }
 }
 
-Context::ListPlan& Context::get_list_plan(const StageProblem& p) {
+// form LIST_STAGE: volume and flux terms in one set of phases, in the storage
+// of `precision`; LIST_OPS: as separate operators in FP64.
+Context::ListPlan& Context::get_list_plan(ListForm form) {
+  const bool ops = form == LIST_OPS;
   std::vector<std::vector<int>> lus;
   const std::vector<std::vector<int>> dims = transform_orders(D, lus);
   const int nord = static_cast<int>(dims.size());
   if (E() > list_ecap) {
     not_recording("stage buffers");
     list_ecap = (E() + E() / 4 + 1023) / 1024 * 1024;
-    list_plan.reset();
+    for (auto& q : list_plans) q.reset();
   }
   u_next.ensure(static_cast<size_t>(E()) * K);
-  auto bits = [](double v) {
-    uintptr_t b;
-    std::memcpy(&b, &v, sizeof b);
-    return b;
-  };
+  const bool f32 = !ops && precision == 1;
   auto ptr = [](const void* q) { return reinterpret_cast<uintptr_t>(q); };
   const double* pen_coef = inst_alpha.empty() ? nullptr : d_pen_coef.p;
-  std::vector<uintptr_t> key = {static_cast<uintptr_t>(same_flux), static_cast<uintptr_t>(is_varcoef(p.flux_kind)),
-                                static_cast<uintptr_t>(interp), static_cast<uintptr_t>(precision), ptr(t_pt.p),
+  std::vector<uintptr_t> key = {static_cast<uintptr_t>(same_flux), static_cast<uintptr_t>(is_varcoef(flux_kind)),
+                                static_cast<uintptr_t>(interp), static_cast<uintptr_t>(f32), ptr(t_pt.p),
                                 ptr(t_la_uv.p), ptr(t_la_uvx.p), ptr(t_la_flx.p), ptr(fucoe.p), ptr(fucoe32.p),
                                 ptr(list_tmp.p), ptr(pen_coef), pen_coef ? static_cast<uintptr_t>(B()) : 0};
   for (int d = 0; d < D; ++d) {
-    key.push_back(bits(p.alpha[d]));
     for (int q = LIST_PT; q <= LIST_FLX; ++q) {
       key.push_back(ptr(l_meta[q * D + d].p));
       key.push_back(ptr(l_ent[q * D + d].p));
     }
   }
+  std::shared_ptr<ListPlan>& list_plan = list_plans[form];
   if (list_plan && list_plan->key == key) return *list_plan;
   not_recording("stage plan");
   HostTimer timer(*this, HOST_PLAN);
-  const bool f32 = precision == 1;
   const double w = f32 ? 4.0 : 8.0;
   list_plan.reset(new ListPlan());
   ListPlan& pl = *list_plan;
@@ -285,10 +284,10 @@ Context::ListPlan& Context::get_list_plan(const StageProblem& p) {
   }
   build(chains, k + 1, m + 1, pl.up, pl.up_final);
   const int nc = same_flux ? 1 : D;
-  pl.up_final.bytes += w * P * (1 + nc) + (is_varcoef(p.flux_kind) ? 8.0 * P * nc : 0.);
+  pl.up_final.bytes += w * P * (1 + nc) + (is_varcoef(flux_kind) ? 8.0 * P * nc : 0.);
   chains.clear();
   // in the reference order: volume terms for d = 0..D-1, then flux terms
-  for (int ft = 0; ft < 2; ++ft)
+  for (int ft = 0; ft < 2; ++ft) {
     for (int d = 0; d < D; ++d)
       for (int o = 0; o < nord; ++o) {
         Chain c{};
@@ -303,13 +302,19 @@ Context::ListPlan& Context::get_list_plan(const StageProblem& p) {
         }
         chains.push_back(c);
       }
-  build(chains, m + 1, k + 1, pl.rhs, pl.rhs_final);
+    if (ops) {
+      build(chains, m + 1, k + 1, ft ? pl.flx : pl.rhs, ft ? pl.flx_final : pl.rhs_final);
+      chains.clear();
+    }
+  }
+  if (!ops) build(chains, m + 1, k + 1, pl.rhs, pl.rhs_final);
   pl.rhs_final.bytes += 8.0 * K * (1 + 3 + D);
+  pl.pen = static_cast<int>(flat.size());
   // the LF penalty stays FP64 in every precision
   int ksz[kMaxDim];
   for (int d = 0; d < D; ++d) ksz[d] = k + 1;
   for (int d = 0; d < D; ++d) {
-    flat.push_back(make_term(LIST_FLX, nullptr, nullptr, 0, ksz, ksz, d, t_aa[4].p, LU_FULL, -p.alpha[d] / 2., false));
+    flat.push_back(make_term(LIST_FLX, nullptr, nullptr, 0, ksz, ksz, d, t_aa[4].p, LU_FULL, 0., false));
     if (pen_coef) flat.back().coef_inst = pen_coef + static_cast<size_t>(d) * B();
   }
   list_tmp.ensure(std::max<size_t>(tmp_most * list_ecap, 1));
@@ -328,9 +333,18 @@ Context::ListPlan& Context::get_list_plan(const StageProblem& p) {
 }
 
 template <class T>
-void Context::stage_list(const StageProblem& p, int scheme, int stage, double dt) {
+void Context::list_phases(const ListPlan& pl, const std::vector<ListPhase>& phases, int cat, int pf1, int pt1) {
+  for (const ListPhase& ph : phases) {
+    prof_begin(cat, ph.bytes * E());
+    list_phase<T>(pf1, pt1, pl.terms.p + ph.first, ph.n, E(), ph.R, u.p, stream);
+    prof_end();
+  }
+}
+
+template <class T>
+void Context::stage_list(const StageProblem& p, int scheme, int stage, double dt, bool first) {
   ensure_lists(LIST_PT, 3, nullptr);
-  ListPlan& pl = get_list_plan(p);
+  ListPlan& pl = get_list_plan(LIST_STAGE);
   constexpr bool f32 = sizeof(T) == 4;
   const int up_kind = interp == 1 ? -1 : p.flux_kind;
   const int ncomp = same_flux ? 1 : D;
@@ -339,18 +353,10 @@ void Context::stage_list(const StageProblem& p, int scheme, int stage, double dt
   if constexpr (f32) { upp = up32.p; fpp = fp32.p; }
   else { upp = up.p; fpp = fp.p; }
   const int64_t n = E();
-  auto phases = [&](const std::vector<ListPlan::Phase>& phs, int cat, int pf1, int pt1) {
-    for (const ListPlan::Phase& ph : phs) {
-      prof_begin(cat, ph.bytes * n);
-      list_phase<T>(pf1, pt1, pl.terms.p + ph.first, ph.n, n, ph.R, u.p, stream);
-      ++stage_launches;
-      prof_end();
-    }
-  };
-  phases(pl.up, PROF_SWEEP, k + 1, m + 1);
+  list_phases<T>(pl, pl.up, PROF_SWEEP, k + 1, m + 1);
   prof_begin(PROF_FLUX, pl.up_final.bytes * n);
-  list_up_final<T>(k + 1, m + 1, pl.terms.p + pl.up_final.first, pl.up_final.n, n, P, u.p, upp, fpp, vcoef.p,
-                   up_kind, p.flux_param, ncomp, stream);
+  list_up_final<T>(k + 1, m + 1, pl.terms.p + pl.up_final.first, pl.up_final.n, n, P, u.p, upp, fpp, vcoef.p, up_kind,
+                   p.flux_param, ncomp, stream);
   ++stage_launches;
   if (interp == 1) {
     flux_herm<T>(upp, fpp, p.flux_kind, T(p.flux_param), ncomp);
@@ -359,18 +365,137 @@ void Context::stage_list(const StageProblem& p, int scheme, int stage, double dt
   prof_end();
   if constexpr (f32) surplus_transform32(fp32.p, fucoe32.p, interA32.p, interB32.p, ncomp);
   else surplus_transform(fp.p, fucoe.p, interA.p, interB.p, ncomp);
-  stage_launches += D;
-  phases(pl.rhs, PROF_RHS_PHASE, m + 1, k + 1);
+  stage_launches += D + static_cast<int64_t>(pl.up.size() + pl.rhs.size());
+  list_phases<T>(pl, pl.rhs, PROF_RHS_PHASE, m + 1, k + 1);
   prof_begin(PROF_RK, pl.rhs_final.bytes * n);
-  list_rhs_final<T>(m + 1, k + 1, pl.terms.p + pl.rhs_final.first, pl.rhs_final.n, D, n, K, rhs.p, u.p, tn.p,
-                    u_next.p, scheme, stage, dt, use_inst_dt ? d_inst_dt.p : nullptr, err_flag.p, stream);
+  list_rhs_final<T>(m + 1, k + 1, pl.terms.p + pl.rhs_final.first, pl.rhs_final.n, D, n, K,
+                    list_rhs(false, scheme, stage, dt, first, p.alpha), stream);
   ++stage_launches;
   prof_end();
   std::swap(u.p, u_next.p);
   std::swap(u.cap, u_next.cap);
 }
 
-template void Context::stage_list<double>(const StageProblem&, int, int, double);
-template void Context::stage_list<float>(const StageProblem&, int, int, double);
+// Arguments of a last-sweep launch that ends in an RK stage.
+ListRhs Context::list_rhs(bool add, int scheme, int stage, double dt, bool first, const double* alpha) const {
+  ListRhs r{rhs.p, add, u.p, u_next.p, first ? u.p : tn.p, first ? tn.p : nullptr, scheme, stage, dt,
+            use_inst_dt ? d_inst_dt.p : nullptr, err_flag.p, {}};
+  for (int d = 0; d < D; ++d) r.coef[d] = alpha ? -alpha[d] / 2. : 1.0;
+  return r;
+}
+
+template void Context::stage_list<double>(const StageProblem&, int, int, double, bool);
+template void Context::stage_list<float>(const StageProblem&, int, int, double, bool);
+
+// ---- the single operators on lists (FP64) ----
+// A partial-sum operator is its phases and one launch that adds the terms of
+// an output in order: D launches where the sweep-by-sweep form takes
+// D 2^(D-1) per term (2D: 28 launches of a right-hand side and stage become
+// 12).  The sums are the same: the sweep-by-sweep form adds term after term to
+// the output as well.
+
+bool Context::list_ops_fit() const {
+  // (Lagrange degree 5 has no list kernels)
+  return m <= 4 && list_stage_fits();
+}
+
+void Context::eval_up_op() {
+  if (!list_ops_fit()) { eval_up(); return; }
+  ensure_lists(LIST_PT, 3, nullptr);
+  const ListPlan& pl = get_list_plan(LIST_OPS);
+  list_phases<double>(pl, pl.up, PROF_SWEEP, k + 1, m + 1);
+  prof_begin(PROF_SWEEP, pl.up_final.bytes * E());
+  list_up_final<double>(k + 1, m + 1, pl.terms.p + pl.up_final.first, pl.up_final.n, E(), P, u.p, up.p, fp.p, vcoef.p, -1,
+                        0., 0, stream);
+  prof_end();
+}
+
+void Context::rhs_lagr_op(bool flux_term) {
+  if (!list_ops_fit()) { rhs_lagr(flux_term); return; }
+  ensure_lists(LIST_PT, 3, nullptr);
+  const ListPlan& pl = get_list_plan(LIST_OPS);
+  const ListPhase& last = flux_term ? pl.flx_final : pl.rhs_final;
+  list_phases<double>(pl, flux_term ? pl.flx : pl.rhs, PROF_RHS_PHASE, m + 1, k + 1);
+  ListRhs r = list_rhs(true, 0, 0, 0., false, nullptr);
+  r.u_next = nullptr;
+  prof_begin(PROF_SWEEP, last.bytes * E());
+  list_rhs_final<double>(m + 1, k + 1, pl.terms.p + last.first, last.n, 0, E(), K, r, stream);
+  prof_end();
+}
+
+void Context::rhs_penalty_op(const double* alpha) {
+  if (!list_ops_fit()) { rhs_penalty(alpha); return; }
+  ensure_lists(LIST_PT, 3, nullptr);
+  const ListPlan& pl = get_list_plan(LIST_OPS);
+  ListRhs r = list_rhs(true, 0, 0, 0., false, alpha);
+  r.u_next = nullptr;
+  prof_begin(PROF_SWEEP, 8.0 * E() * K * (2 + D));
+  list_rhs_final<double>(m + 1, k + 1, pl.terms.p + pl.pen, 0, D, E(), K, r, stream);
+  prof_end();
+}
+
+// The assembled constant-coefficient operator as D sweeps of one launch: added
+// to the right-hand side, or with a whole RK stage (run = true).
+void Context::linear_list(const double* coef, bool run, int scheme, int stage, double dt, bool first) {
+  linear_tables(coef);
+  ensure_lists(LIST_LIN, 1, nz_lin.p);
+  u_next.ensure(static_cast<size_t>(E()) * K);
+  std::vector<uintptr_t> key = {reinterpret_cast<uintptr_t>(l_meta[LIST_LIN * D].p)};
+  for (int d = 0; d < D; ++d)
+    for (const void* q : {static_cast<const void*>(l_meta[LIST_LIN * D + d].p), static_cast<const void*>(l_ent[LIST_LIN * D + d].p),
+                          static_cast<const void*>(t_lin[d].p)})
+      key.push_back(reinterpret_cast<uintptr_t>(q));
+  std::shared_ptr<ListPlan>& pl = list_plans[LIST_LINEAR];
+  if (!pl || pl->key != key) {
+    pl.reset(new ListPlan());
+    std::vector<ListTerm> terms;
+    std::vector<int2> rofs;
+    const int k1 = k + 1, R = K / k1;
+    for (int d = 0; d < D; ++d) {
+      ListTerm t{};
+      t.M = t_lin[d].p; t.meta = l_meta[LIST_LIN * D + d].p; t.ent = l_ent[LIST_LIN * D + d].p;
+      t.coef = 1.0; t.comp_size = t.Tin = t.Tout = K; t.R = R; t.ns = 1 << nmax; t.lu = LU_FULL;
+      t.sdd = 1;
+      for (int q = d + 1; q < D; ++q) t.sdd *= k1;
+      t.sod = t.sdd;
+      terms.push_back(t);
+      for (int r = 0; r < R; ++r) {
+        const int o = (r / t.sdd) * t.sdd * k1 + r % t.sdd;
+        rofs.push_back(int2{o, o});
+      }
+    }
+    upload(pl->rofs, rofs, stream);
+    for (int d = 0; d < D; ++d) terms[d].rofs = pl->rofs.p + static_cast<size_t>(d) * R;
+    upload(pl->terms, terms, stream);
+    sync();
+    pl->key = key;
+  }
+  ListRhs r = list_rhs(!run, scheme, stage, dt, first, nullptr);
+  if (!run) r.u_next = nullptr;
+  prof_begin(PROF_SWEEP, 8.0 * E() * K * (run ? D + 4 : D + 2));
+  list_rhs_final<double>(k + 1, k + 1, pl->terms.p, 0, D, E(), K, r, stream);
+  prof_end();
+  if (run) {
+    std::swap(u.p, u_next.p);
+    std::swap(u.cap, u_next.cap);
+  }
+}
+
+// One RK stage of du/dt = A u; first: u^n <- u before it.
+void Context::linear_stage(const double* coef, int scheme, int stage, double dt, bool first) {
+  if (list_stage_fits()) {
+    linear_list(coef, true, scheme, stage, dt, first);
+    return;
+  }
+  if (first) rk_init();
+  rhs_zero();
+  rhs_linear(coef);
+  rk_stage(scheme, stage, dt);
+}
+
+void Context::rhs_linear_op(const double* coef) {
+  if (list_stage_fits()) linear_list(coef, false, 0, 0, 0., false);
+  else rhs_linear(coef);
+}
 
 }  // namespace adg

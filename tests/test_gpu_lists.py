@@ -1,14 +1,15 @@
 """The stage on source lists (the form that runs when no mapping is fixed)
 against the fused per-element kernels and the per-sweep path, bit for bit:
 every basis size the fused stage provides, both interpolation families, the
-level-sum cap, FP32 storage, and grids on both sides of the size at which the
+level-sum cap, FP32 storage, the single operators, and grids on both sides of the size at which the
 kernels request more sources at a time (16,384 elements)."""
 import numpy as np
 import pytest
 
 import pyadg
+import pyoracle
 import workloads
-from common import first_diff, ic_params, problem
+from common import first_diff, ic_params, init_both, oracle_run_linear, problem
 
 pytestmark = pytest.mark.gpu
 
@@ -70,3 +71,34 @@ def test_few_and_many_elements(batch):
     _same(_steps(s, p, -1, 1), _steps(s, p, 3, 1), "fixed grid")
     # refinement and coarsening grow and shrink the lists
     _same(_steps(s, ws[0].problem, -1, 2), _steps(s, ws[0].problem, 3, 2), "adaptive")
+
+
+@pytest.mark.parametrize("dim,k,m,cap", [(1, 1, 2, -1), (2, 3, 3, -1), (3, 2, 3, 3), (4, 1, 2, -1)])
+def test_single_operators_match_oracle(dim, k, m, cap):
+    """Operators on lists, added to what the right-hand side holds, against
+    the oracle; the constant-coefficient operator with both signs of speed."""
+    print(f"[case] list operators dim={dim} k={k} m={m} cap={cap}", flush=True)
+    nmax = 5 if dim < 3 else 4
+    g = pyadg.Solution(dim, k, m, nmax, True, nmax)
+    o = pyoracle.Oracle(dim, k, m, nmax, True, nmax)
+    init_both(g, o, ic_params(1, shift=0.21), 1e10)
+    speeds, alpha = [0.7, -1.3, 0.4, -0.2][:dim], [1.2, 0.9, 1.1, 0.8][:dim]
+    for s in (g, o):
+        s.set_level_sum_cap(cap)
+        s.eval_up()
+        s.flux(pyadg.FLUX_VARCOEF, [0.3])
+        s.fp_to_coe()
+        s.rhs_zero()
+        s.rhs_linear(speeds)
+        s.rhs_lagr_vol()
+        s.rhs_lagr_flx()
+        s.rhs_penalty(alpha)
+        s.rhs_penalty([2 * a for a in alpha])
+    for field in (pyadg.FIELD_UP, pyadg.FIELD_RHS):
+        a, b = g.get(field), o.get(field)
+        assert np.array_equal(a, b), f"field {field}: " + first_diff(a, b)
+    g.run_linear(speeds, 1e-3, 2)
+    oracle_run_linear(o, speeds, 1e-3, 2)
+    for field in (pyadg.FIELD_UCOE, pyadg.FIELD_RHS, pyadg.FIELD_TN):
+        a, b = g.get(field), o.get(field)
+        assert np.array_equal(a, b), f"field {field}: " + first_diff(a, b)
