@@ -457,6 +457,8 @@ class Context {
   void proposer_features(const std::vector<double>& eps, float* feats_dev, int32_t* leaf_dev);
   DevBuf<float> prop_params, prop_grad, prop_m1, prop_m2, prop_norm, prop_feats, prop_prob;
   DevBuf<float> prop_h1, prop_h2, prop_dh1, prop_dh2, prop_dz, prop_x, prop_y, prop_w, prop_loss;
+  DevBuf<float> prop_part;  // gradient sums of the sample chunks
+  void proposer_grad(const int32_t* idx, int64_t n, float scale);
   DevBuf<uint16_t> prop_params16;  // FP16 copy for inference
   DevBuf<int32_t> prop_leaf, prop_idx;
   DevBuf<double> prop_eps;
