@@ -325,16 +325,15 @@ class Context {
   void rhs_linear_op(const double* coef);
   void linear_stage(const double* coef, int scheme, int stage, double dt, bool first);
   void linear_list(const double* coef, bool run, int scheme, int stage, double dt, bool first);
-  void linear_tables(const double* coef);  // t_lin and nz_lin for these speeds
-  DevBuf<uint8_t> nz_lin;
+  void linear_tables(const double* coef);  // t_lin and its pairs for these speeds
   template <class T>
   void flux_herm(const T* up, T* fp, int kind, T s, int ncomp);
   // lists of the given kinds for the current grid, level-sum cap and
-  // interpolation family (nz: which table blocks count, default nz_tab)
-  void ensure_lists(int kind0, int nkind, const uint8_t* nz);
+  // interpolation family
+  void ensure_lists(int kind0, int nkind);
   void list_nonzero_tables();
   static constexpr int kListKinds = 4;
-  DevBuf<uint8_t> nz_tab;
+  DevBuf<uint32_t> nz_tab[kListKinds];  // pairs of each kind (list_nonzero)
   int nz_interp = -1;
   DevBuf<int4> l_meta[kListKinds * kMaxDim];
   DevBuf<int2> l_ent[kListKinds * kMaxDim];

@@ -1132,12 +1132,12 @@ void Context::linear_tables(const double* coef) {
   if (lin_coef.size() == static_cast<size_t>(D) && std::equal(lin_coef.begin(), lin_coef.end(), coef)) return;
   const int ns = 1 << nmax, kb = (k + 1) * (k + 1);
   const int64_t n = static_cast<int64_t>(ns) * ns * kb;
-  nz_lin.ensure(static_cast<size_t>(ns) * ns);
+  nz_tab[LIST_LIN].ensure(static_cast<size_t>(ns) * ((ns + 31) / 32));
   for (int d = 0; d < D; ++d) {
     t_lin[d].ensure(static_cast<size_t>(n));
     hipLaunchKernelGGL(k_linear_table, dim3(nblocks(n)), dim3(kBlock), 0, stream, t_aa[1].p,
                        coef[d] >= 0 ? t_aa[2].p : t_aa[3].p, coef[d], t_lin[d].p, n);
-    list_nonzero(nz_lin.p, t_lin[d].p, ns, kb, LIST_LIN, d == 0, stream);
+    list_nonzero(nz_tab[LIST_LIN].p, t_lin[d].p, ns, kb, false, d == 0, stream);
   }
   lin_coef.assign(coef, coef + D);
   list_version[LIST_LIN] = -1;

@@ -54,7 +54,8 @@ struct ListBuildArgs {
   const uint32_t* fbits[kMaxDimK];
   const int32_t* lsum;
   const int32_t* inst;
-  const uint8_t* nz;  // [target slot * ns + source slot]: bit per ListKind
+  // pairs of each kind: rows of ns bits (whole words) per target slot
+  const uint32_t* nz[LIST_KINDS];
   int4* meta[LIST_KINDS * kMaxDimK];  // [kind * D + d]; null: not built
   int2* ent[LIST_KINDS * kMaxDimK];
   int64_t cap[LIST_KINDS * kMaxDimK];  // entries that fit
@@ -64,9 +65,11 @@ struct ListBuildArgs {
   int D, ns, level_cap;
 };
 void list_fill_totals(int32_t* total, int n, hipStream_t s);  // zeroes the counters
-void list_build(const ListBuildArgs& a, int kind0, int nkind, hipStream_t s);
-// bit of `kind` in nz wherever a block of M is not zero (or: every block)
-void list_nonzero(uint8_t* nz, const double* M, int ns, int block, int kind, bool clear, hipStream_t s);
+// lmax: deepest level of the grid in any dimension
+void list_build(const ListBuildArgs& a, int kind0, int nkind, int lmax, hipStream_t s);
+// sets the bit of every pair whose block of M is not zero (no M: every pair),
+// among nested cells only when in_support
+void list_nonzero(uint32_t* nz, const double* M, int ns, int block, bool in_support, bool clear, hipStream_t s);
 
 // ---- sweeps ----
 // term values of a block of a final kernel, kept in LDS

@@ -18,89 +18,152 @@ inline unsigned nblocks(int64_t n) { return static_cast<unsigned>((n + kBlock - 
 // ---------------------------------------------------------------------------
 // build
 
-__global__ __launch_bounds__(kBlock) void k_list_nz(uint8_t* nz, const double* M, int64_t n, int block, int bit,
-                                                    int clear) {
+// Whether the cells of two slots are nested (their supports overlap).
+__device__ __forceinline__ bool nested(int a, int b) {
+  const int la = slot_level(a), lb = slot_level(b);
+  if (la <= 1 || lb <= 1) return true;
+  return la >= lb ? (a >> (la - lb)) == b : (b >> (lb - la)) == a;
+}
+
+__global__ __launch_bounds__(kBlock) void k_list_nz(uint32_t* nz, const double* M, int ns, int nw, int block,
+                                                    int in_support) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  if (i >= static_cast<int64_t>(ns) * ns) return;
+  const int st = static_cast<int>(i / ns), s = static_cast<int>(i % ns);
   bool any = M == nullptr;
   if (M)
     for (int j = 0; j < block; ++j) any = any || M[i * block + j] != 0.;
-  uint8_t v = nz[i];
-  if (clear) v &= static_cast<uint8_t>(~bit);
-  nz[i] = any ? static_cast<uint8_t>(v | bit) : v;
+  if (any && (!in_support || nested(st, s))) atomicOr(&nz[st * nw + (s >> 5)], 1u << (s & 31));
+}
+
+__global__ __launch_bounds__(kBlock) void k_list_clear(uint32_t* nz, int64_t n) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i < n) nz[i] = 0;
 }
 
 __global__ void k_list_zero(int32_t* p, int n) {
   if (static_cast<int>(threadIdx.x) < n) p[threadIdx.x] = 0;
 }
 
-// Present sources of element e along dimension d for the lists of one kind,
-// ascending: f(source element, source slot).
-template <class F>
-__device__ __forceinline__ void list_sources(const ListBuildArgs& a, int kind, int d, int64_t e, int st, F&& f) {
-  const int fb = a.fbase[d][e];
-  int maxl = a.fmaxl[d][e];
-  if (a.level_cap >= 0) {  // coarse grid (FastMultiplyLU::transform_1D_coarse_grid)
-    const int ls = a.lsum[e];
-    if (ls > a.level_cap) return;
-    maxl = min(maxl, a.level_cap - ls + slot_level(st));
-  }
-  const int32_t* fmap = a.fmap[d];
-  const uint8_t* nz = a.nz + static_cast<int64_t>(st) * a.ns;
-  const bool flx = kind == LIST_FLX || kind == LIST_LIN;
-  for_each_present(st, maxl, flx, LU_FULL, a.fbits[d], fb, [&](int s) {
-    if (!(nz[s] >> kind & 1)) return;
-    const int src = fmap[fb + s];
-    if (src >= 0) f(src, s);
-  });
-}
+// G threads per (dimension, target) for up to three kinds of lists at once.
+// The sources of a target are the set bits of (occupancy of its fiber) AND (the
+// target slot's row of nonzero pairs), in slot order; each thread counts and
+// later writes those of its run of 16-cell pieces, so the threads of a block in
+// order hold the block's entries in order.  The block takes room for them with
+// one atomic add per list.  Where a target's entries lie differs from run to
+// run, what they hold does not.
+// Bound: latency of the bit words and the fiber map.  Walking the relation a
+// cell at a time, a thread per (list, target): 590 us for 237 thousand elements
+// of the rotating wave at level 9 (the coarse targets' walks), 168 us for 90 to
+// 165 thousand of 512 Burgers solves, 68 us for 145 elements; a thread per
+// target over words 747, 54 and 24 us; now 118, 29 and 11 us.
+constexpr int kPiece = 16;
 
-// Thread per (kind, dimension, target): counts its sources, takes room for
-// the block's sources with one atomic add, and writes them.  Where a target's
-// entries lie differs from run to run, what they hold does not.
-__global__ __launch_bounds__(kBlock) void k_list_build(ListBuildArgs a, int kind0) {
-  __shared__ int s_wave[kBlock / kWave];
-  __shared__ int s_base;
-  const int kind = kind0 + static_cast<int>(blockIdx.y) / a.D, d = static_cast<int>(blockIdx.y) % a.D;
-  const int list = kind * a.D + d;
-  const int64_t e = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  int n = 0, nu = 0, st = 0;
+template <int G>
+__global__ __launch_bounds__(kBlock) void k_list_build(ListBuildArgs a, int kind0, int nkind) {
+  constexpr int NK = 3;
+  __shared__ int s_wave[NK][kBlock / kWave];
+  __shared__ int s_base[NK];
+  const int d = blockIdx.y;
+  const int64_t e = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / G;
+  const int g = threadIdx.x % G, lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  const int32_t* fmap = a.fmap[d];
+  const int nw = (a.ns + 31) / 32;
+  int st = 0, fb = 0, maxl = -1, lt = 0;
   if (e < a.E) {
     st = a.slot[d][e];
-    const int lt = slot_level(st);
-    list_sources(a, kind, d, e, st, [&](int, int s) {
-      ++n;
-      nu += slot_level(s) <= lt;
-    });
+    lt = slot_level(st);
+    fb = a.fbase[d][e];
+    maxl = a.fmaxl[d][e];
+    if (a.level_cap >= 0) {  // coarse grid (FastMultiplyLU::transform_1D_coarse_grid)
+      const int ls = a.lsum[e];
+      maxl = ls > a.level_cap ? -1 : min(maxl, a.level_cap - ls + lt);
+    }
   }
-  int inc = n;  // inclusive sum over the wavefront
-  for (int o = 1; o < kWave; o <<= 1) {
-    const int v = __shfl_up(inc, o);
-    if (lane >= o) inc += v;
+  // the cells of levels 0 .. maxl are the slots below 2^maxl
+  const int cells = maxl < 0 ? 0 : 1 << maxl;
+  const int per = ((cells + kPiece - 1) / kPiece + G - 1) / G;  // pieces of a thread
+  const int p0 = g * per, p1 = min(p0 + per, (cells + kPiece - 1) / kPiece);
+  const uint32_t* occ = a.fbits[d] + (fb >> 5);
+  const int64_t row = static_cast<int64_t>(st) * nw;
+  // present cells of piece p (a fiber of fewer than 32 cells shares its word)
+  auto present = [&](int p) {
+    const uint32_t m = (occ[p >> 1] >> (fb & 31)) >> (p & 1) * kPiece & 0xffffu;
+    return cells < (p + 1) * kPiece ? m & ((1u << max(cells - p * kPiece, 0)) - 1u) : m;
+  };
+  auto pairs = [&](int q, int p) { return a.nz[kind0 + q][row + (p >> 1)] >> (p & 1) * kPiece; };
+  int n[NK] = {0, 0, 0}, nu[NK] = {0, 0, 0};
+  for (int p = p0; p < p1; ++p) {
+    const uint32_t m = present(p);
+    // slots of levels up to lt: below 2^lt
+    const int up_cells = (1 << lt) - p * kPiece;
+    const uint32_t up = up_cells >= kPiece ? 0xffffu : (up_cells <= 0 ? 0u : (1u << up_cells) - 1u);
+#pragma unroll
+    for (int q = 0; q < NK; ++q)
+      if (q < nkind) {
+        const uint32_t mq = m & pairs(q, p);
+        n[q] += __popc(mq);
+        nu[q] += __popc(mq & up);
+      }
   }
-  if (lane == kWave - 1) s_wave[wave] = inc;
+  int beg[NK], all[NK];
+#pragma unroll
+  for (int q = 0; q < NK; ++q) {
+    int inc = n[q];  // inclusive sum over the wavefront
+    for (int o = 1; o < kWave; o <<= 1) {
+      const int v = __shfl_up(inc, o);
+      if (lane >= o) inc += v;
+    }
+    if (lane == kWave - 1) s_wave[q][wave] = inc;
+    beg[q] = inc - n[q];
+    all[q] = __shfl(inc, lane - g + G - 1) - __shfl(beg[q], lane - g);
+    for (int o = 1; o < G; o <<= 1) nu[q] += __shfl_xor(nu[q], o);
+  }
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (static_cast<int>(threadIdx.x) < nkind) {
+    const int q = threadIdx.x;
     int sum = 0;
     for (int w = 0; w < kBlock / kWave; ++w) {
-      const int v = s_wave[w];
-      s_wave[w] = sum;
+      const int v = s_wave[q][w];
+      s_wave[q][w] = sum;
       sum += v;
     }
-    s_base = atomicAdd(&a.total[list], sum);
+    s_base[q] = atomicAdd(&a.total[(kind0 + q) * a.D + d], sum);
   }
   __syncthreads();
   if (e >= a.E) return;
-  int beg = s_base + s_wave[wave] + inc - n;
-  if (static_cast<int64_t>(beg) + n > a.cap[list]) {  // (the bound of the host is exceeded: never)
-    atomicOr(a.err, ERR_COOP);
-    a.meta[list][e] = make_int4(0, 0, st, a.inst[e]);
-    return;
+  for (int q = 0; q < nkind; ++q) {
+    const int list = (kind0 + q) * a.D + d;
+    int at = beg[q] + s_base[q] + s_wave[q][wave], left = n[q];
+    if (static_cast<int64_t>(at) + left > a.cap[list]) {  // (the host's bound is exceeded: never)
+      atomicOr(a.err, ERR_COOP);
+      left = all[q] = 0;
+    }
+    if (g == 0) a.meta[list][e] = make_int4(all[q] ? at : 0, all[q] ? nu[q] | all[q] << 16 : 0, st, a.inst[e]);
+    int2* ent = a.ent[list];
+    int p = p0;
+    uint32_t m = left > 0 ? present(p) & pairs(q, p) : 0;
+    for (; left > 0; left -= 4, at += 4) {  // four sources at a time
+      int s[4], src[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        s[j] = s[0];
+        if (j < left) {
+          while (!m) {
+            ++p;
+            m = present(p) & pairs(q, p);
+          }
+          s[j] = kPiece * p + __builtin_ctz(m);
+          m &= m - 1;
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) src[j] = fmap[fb + s[j]];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (j < left) ent[at + j] = make_int2(src[j], s[j]);
+    }
   }
-  a.meta[list][e] = make_int4(beg, nu | n << 16, st, a.inst[e]);
-  int2* ent = a.ent[list];
-  list_sources(a, kind, d, e, st, [&](int src, int s) { ent[beg++] = make_int2(src, s); });
 }
 
 // ---------------------------------------------------------------------------
@@ -381,18 +444,27 @@ void rhs_final_t(const ListTerm* terms, int nterm, int npen, int64_t E, int K, c
 
 }  // namespace
 
-void list_nonzero(uint8_t* nz, const double* M, int ns, int block, int kind, bool clear, hipStream_t s) {
+void list_nonzero(uint32_t* nz, const double* M, int ns, int block, bool in_support, bool clear, hipStream_t s) {
   const int64_t n = static_cast<int64_t>(ns) * ns;
-  hipLaunchKernelGGL(k_list_nz, dim3(nblocks(n)), dim3(kBlock), 0, s, nz, M, n, block, 1 << kind, clear ? 1 : 0);
+  const int nw = (ns + 31) / 32;
+  if (clear) hipLaunchKernelGGL(k_list_clear, dim3(nblocks(int64_t{ns} * nw)), dim3(kBlock), 0, s, nz, int64_t{ns} * nw);
+  hipLaunchKernelGGL(k_list_nz, dim3(nblocks(n)), dim3(kBlock), 0, s, nz, M, ns, nw, block, in_support ? 1 : 0);
 }
 
 void list_fill_totals(int32_t* total, int n, hipStream_t s) {
   hipLaunchKernelGGL(k_list_zero, dim3(1), dim3(kWave), 0, s, total, n);
 }
 
-void list_build(const ListBuildArgs& a, int kind0, int nkind, hipStream_t s) {
-  if (a.E > 0)
-    hipLaunchKernelGGL(k_list_build, dim3(nblocks(a.E), nkind * a.D), dim3(kBlock), 0, s, a, kind0);
+void list_build(const ListBuildArgs& a, int kind0, int nkind, int lmax, hipStream_t s) {
+  if (a.E == 0) return;
+  // more threads a target where fibers are long, or where the grid is small and
+  // a thread's chain of loads is the launch's time
+  if (lmax <= 7 && a.E > kFewElements)
+    hipLaunchKernelGGL(k_list_build<2>, dim3(nblocks(a.E * 2), a.D), dim3(kBlock), 0, s, a, kind0, nkind);
+  else if (lmax <= 8)
+    hipLaunchKernelGGL(k_list_build<4>, dim3(nblocks(a.E * 4), a.D), dim3(kBlock), 0, s, a, kind0, nkind);
+  else
+    hipLaunchKernelGGL(k_list_build<8>, dim3(nblocks(a.E * 8), a.D), dim3(kBlock), 0, s, a, kind0, nkind);
 }
 
 template <class T>

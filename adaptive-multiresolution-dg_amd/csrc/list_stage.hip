@@ -63,26 +63,22 @@ bool Context::list_stage_fits() const {
 // Tables whose blocks decide which pairs a list holds.
 void Context::list_nonzero_tables() {
   const int ns = 1 << nmax, kb = (k + 1) * (m + 1);
-  nz_tab.ensure(static_cast<size_t>(ns) * ns);
-  // (no table: every block counts)
-  list_nonzero(nz_tab.p, nullptr, ns, 1, LIST_VOL, true, stream);
-  list_nonzero(nz_tab.p, t_pt.p, ns, kb, LIST_PT, true, stream);
-  list_nonzero(nz_tab.p, t_la_flx.p, ns, kb, LIST_FLX, true, stream);
-  list_nonzero(nz_tab.p, t_aa[4].p, ns, (k + 1) * (k + 1), LIST_FLX, false, stream);
+  for (int q = LIST_PT; q <= LIST_FLX; ++q) nz_tab[q].ensure(static_cast<size_t>(ns) * ((ns + 31) / 32));
+  list_nonzero(nz_tab[LIST_VOL].p, nullptr, ns, 1, true, true, stream);
+  list_nonzero(nz_tab[LIST_PT].p, t_pt.p, ns, kb, true, true, stream);
+  list_nonzero(nz_tab[LIST_FLX].p, t_la_flx.p, ns, kb, false, true, stream);
+  list_nonzero(nz_tab[LIST_FLX].p, t_aa[4].p, ns, (k + 1) * (k + 1), false, false, stream);
   nz_interp = interp;
 }
 
-void Context::ensure_lists(int kind0, int nkind, const uint8_t* nz) {
+void Context::ensure_lists(int kind0, int nkind) {
   bool ok = true;
   for (int q = kind0; q < kind0 + nkind; ++q)
     ok = ok && list_version[q] == grid_version && list_level_cap[q] == lsum_cap && list_interp[q] == interp;
   if (ok) return;
   not_recording("source lists");
   HostTimer timer(*this, HOST_UPLOAD);
-  if (!nz) {
-    if (nz_interp != interp) list_nonzero_tables();
-    nz = nz_tab.p;
-  }
+  if (kind0 != LIST_LIN && nz_interp != interp) list_nonzero_tables();
   ListBuildArgs a{};
   for (int d = 0; d < D; ++d) {
     a.slot[d] = g_slot[d].p;
@@ -91,16 +87,19 @@ void Context::ensure_lists(int kind0, int nkind, const uint8_t* nz) {
     a.fmap[d] = g_fmap[d].p;
     a.fbits[d] = g_fbits[d].p;
   }
-  a.lsum = g_lsum.p; a.inst = g_inst.p; a.nz = nz; a.err = err_flag.p;
+  a.lsum = g_lsum.p; a.inst = g_inst.p; a.err = err_flag.p;
   a.E = E(); a.D = D; a.ns = 1 << nmax; a.level_cap = lsum_cap;
+  for (int q = 0; q < LIST_KINDS; ++q) a.nz[q] = nz_tab[q].p;
   l_total.ensure(LIST_KINDS * kMaxDim);
   a.total = l_total.p;
   // An element of level l has at most l + 1 related cells at levels up to its
   // own in a nested relation, 2 l + 3 in one that counts touching cells, and
   // as many pairs (less itself) with it as the finer one are in the L parts.
+  int deepest = 0;
   for (int d = 0; d < D; ++d) {
     int lmax = 0;
     for (int i = 0; i < B(); ++i) lmax = std::max(lmax, inst_lmax[static_cast<size_t>(i) * D + d]);
+    deepest = std::max(deepest, lmax);
     for (int q = kind0; q < kind0 + nkind; ++q) {
       const bool touch = q == LIST_FLX || q == LIST_LIN;
       const int64_t room = E() * (touch ? 4 * lmax + 4 : 2 * lmax + 1);
@@ -113,7 +112,7 @@ void Context::ensure_lists(int kind0, int nkind, const uint8_t* nz) {
     }
   }
   list_fill_totals(l_total.p + kind0 * D, nkind * D, stream);
-  list_build(a, kind0, nkind, stream);
+  list_build(a, kind0, nkind, deepest, stream);
   for (int q = kind0; q < kind0 + nkind; ++q) {
     list_version[q] = grid_version;
     list_level_cap[q] = lsum_cap;
@@ -343,7 +342,7 @@ void Context::list_phases(const ListPlan& pl, const std::vector<ListPhase>& phas
 
 template <class T>
 void Context::stage_list(const StageProblem& p, int scheme, int stage, double dt, bool first) {
-  ensure_lists(LIST_PT, 3, nullptr);
+  ensure_lists(LIST_PT, 3);
   ListPlan& pl = get_list_plan(LIST_STAGE);
   constexpr bool f32 = sizeof(T) == 4;
   const int up_kind = interp == 1 ? -1 : p.flux_kind;
@@ -401,7 +400,7 @@ bool Context::list_ops_fit() const {
 
 void Context::eval_up_op() {
   if (!list_ops_fit()) { eval_up(); return; }
-  ensure_lists(LIST_PT, 3, nullptr);
+  ensure_lists(LIST_PT, 3);
   const ListPlan& pl = get_list_plan(LIST_OPS);
   list_phases<double>(pl, pl.up, PROF_SWEEP, k + 1, m + 1);
   prof_begin(PROF_SWEEP, pl.up_final.bytes * E());
@@ -412,7 +411,7 @@ void Context::eval_up_op() {
 
 void Context::rhs_lagr_op(bool flux_term) {
   if (!list_ops_fit()) { rhs_lagr(flux_term); return; }
-  ensure_lists(LIST_PT, 3, nullptr);
+  ensure_lists(LIST_PT, 3);
   const ListPlan& pl = get_list_plan(LIST_OPS);
   const ListPhase& last = flux_term ? pl.flx_final : pl.rhs_final;
   list_phases<double>(pl, flux_term ? pl.flx : pl.rhs, PROF_RHS_PHASE, m + 1, k + 1);
@@ -425,7 +424,7 @@ void Context::rhs_lagr_op(bool flux_term) {
 
 void Context::rhs_penalty_op(const double* alpha) {
   if (!list_ops_fit()) { rhs_penalty(alpha); return; }
-  ensure_lists(LIST_PT, 3, nullptr);
+  ensure_lists(LIST_PT, 3);
   const ListPlan& pl = get_list_plan(LIST_OPS);
   ListRhs r = list_rhs(true, 0, 0, 0., false, alpha);
   r.u_next = nullptr;
@@ -438,7 +437,7 @@ void Context::rhs_penalty_op(const double* alpha) {
 // to the right-hand side, or with a whole RK stage (run = true).
 void Context::linear_list(const double* coef, bool run, int scheme, int stage, double dt, bool first) {
   linear_tables(coef);
-  ensure_lists(LIST_LIN, 1, nz_lin.p);
+  ensure_lists(LIST_LIN, 1);
   u_next.ensure(static_cast<size_t>(E()) * K);
   std::vector<uintptr_t> key = {reinterpret_cast<uintptr_t>(l_meta[LIST_LIN * D].p)};
   for (int d = 0; d < D; ++d)
