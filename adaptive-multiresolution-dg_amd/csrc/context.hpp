@@ -439,7 +439,7 @@ class Context {
   int64_t vop_blocks = 0, vop_version = -1, vop_nnz_entries = 0, imex_version = -1;
   std::vector<int32_t> vop_key_tid;   // 1D integral key -> table entry
   std::vector<double> vop_tab_host;   // per entry: mass, stiffness ((k+1)^2 each)
-  DevBuf<int32_t> vop_rowptr, vop_col, vop_recptr, vop_rec, cg_state, cg_inst_chunk;
+  DevBuf<int32_t> vop_rowptr, vop_col, vop_recptr, vop_rec, cg_state, cg_inst_chunk, cg_chunk_inst, cg_done;
   DevBuf<double> vop_tab, vop_val, imex_tn, imex_G[4], imex_F[2], cg_b, cg_r, cg_p, cg_t, cg_inv, cg_part, cg_scal;
   DevBuf<int64_t> cg_chunk;
   int cg_nchunk = 0;

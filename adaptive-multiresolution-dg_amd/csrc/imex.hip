@@ -31,6 +31,7 @@
 #include <stdexcept>
 
 #include "context.hpp"
+#include "kern.hpp"
 
 namespace adg {
 
@@ -111,18 +112,27 @@ __global__ __launch_bounds__(kVB) void k_vop_spmv(int64_t n, int K, const int32_
 }
 
 // y = A x (mode 0) or y = (I - c A) x (mode 2): a workgroup per row, the
-// row's entries split over the threads, partial sums added in a fixed tree.
+// row's entries round 256 partial sums, a thread each (two requested at a time),
+// added in a fixed binary tree.  The K rows of an element run on one XCD one
+// after another (they share the cache lines of its blocks), the elements go
+// round the XCDs: coarse ones, first in order, couple with far more columns.
+// Bound: the operator's values (37 MB for 1,018 elements) and the longest rows:
+// 15.6 us; rows round the XCDs and eight barriers of a tree in LDS 21.8; a
+// contiguous range of rows per XCD 25, a workgroup per element 73, a wavefront
+// per row 57.
 constexpr int kWB = 256;
-__global__ __launch_bounds__(kWB) void k_vop_spmv_wide(int K, const int32_t* rowptr, const int32_t* col,
+__global__ __launch_bounds__(kWB) void k_vop_spmv_wide(int64_t E, int K, const int32_t* rowptr, const int32_t* col,
                                                        const double* val, const double* x, double* y, int mode,
                                                        double c) {
   __shared__ double red[kWB];
-  const int64_t r = blockIdx.x;
-  const int64_t e = r / K;
-  const int i = static_cast<int>(r - e * K);
+  const unsigned g = blockIdx.x / kXcds;
+  const int i = static_cast<int>(g % K);
+  const int64_t e = static_cast<int64_t>(g / K) * kXcds + blockIdx.x % kXcds;
+  if (e >= E) return;
   const int b0 = rowptr[e], b1 = rowptr[e + 1];
   const int nent = (b1 - b0) * K;
   double t = 0.;
+#pragma unroll 2
   for (int q = threadIdx.x; q < nent; q += kWB) {
     const int bq = q / K, j = q - bq * K;
     const int b = b0 + bq;
@@ -133,11 +143,14 @@ __global__ __launch_bounds__(kWB) void k_vop_spmv_wide(int K, const int32_t* row
   }
   red[threadIdx.x] = t;
   __syncthreads();
-  for (int w = kWB / 2; w > 0; w /= 2) {
-    if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) y[r] = (mode == 2 && b0 == b1) ? x[r] : red[0];
+  if (threadIdx.x >= 64) return;
+  // sums l, l + 64, l + 128 and l + 192: the tree's first two levels, the rest
+  // across the wavefront
+  const double* s = red + threadIdx.x;
+  double v = (s[0] + s[128]) + (s[64] + s[192]);
+  for (int w = 32; w > 0; w /= 2) v += __shfl_down(v, w);
+  const int64_t r = e * K + i;
+  if (threadIdx.x == 0) y[r] = (mode == 2 && b0 == b1) ? x[r] : v;
 }
 
 // Jacobi preconditioner of I - c A: 1 / diagonal when non-zero, else 1.
@@ -153,20 +166,16 @@ __global__ __launch_bounds__(kVB) void k_vop_invdiag(int64_t n, int K, const int
   inv[r] = (m != 0.) ? 1. / m : 1.;
 }
 
-// Per-chunk partial sums (each chunk lies inside one instance): mode 0 sums
-// a*b into slot 0; mode 1 sums a*a into slot 0 and a*(inv*a) into slot 1.
-__global__ __launch_bounds__(kVB) void k_cg_dot(const int64_t* chunk, const double* a, const double* b,
-                                                const double* inv, int mode, double* part) {
+// Per-chunk partial sums (each chunk lies inside one instance): a*a into slot
+// 0 and a*(inv*a) into slot 1.
+__global__ __launch_bounds__(kVB) void k_cg_dot(const int64_t* chunk, const double* a, const double* inv,
+                                                double* part) {
   __shared__ double s0[kVB], s1[kVB];
   const int64_t lo = chunk[2 * blockIdx.x], hi = chunk[2 * blockIdx.x + 1];
   double t0 = 0., t1 = 0.;
   for (int64_t q = lo + threadIdx.x; q < hi; q += kVB) {
-    if (mode == 0) {
-      t0 += a[q] * b[q];
-    } else {
-      t0 += a[q] * a[q];
-      t1 += a[q] * (inv[q] * a[q]);
-    }
+    t0 += a[q] * a[q];
+    t1 += a[q] * (inv[q] * a[q]);
   }
   s0[threadIdx.x] = t0;
   s1[threadIdx.x] = t1;
@@ -225,35 +234,6 @@ __global__ __launch_bounds__(kVB) void k_cg_start(int64_t n, const double* b, co
   p[q] = inv[q] * b[q];
 }
 
-// x += alpha p, r -= alpha t with alpha = absNew / p.Mp of the row's instance
-__global__ __launch_bounds__(kVB) void k_cg_update(int64_t n, int K, const int32_t* inst, const int32_t* state,
-                                                   const double* scal, const double* p, const double* t, double* x,
-                                                   double* r) {
-  const int64_t q = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (q >= n) return;
-  const int i = inst[q / K];
-  if (!state[2 * i]) return;
-  const double alpha = scal[i * kS + 2] / scal[i * kS + 6];
-  x[q] += alpha * p[q];
-  r[q] -= alpha * t[q];
-}
-
-// after the residual dots: converged, or beta and the next absNew
-__global__ void k_cg_step(int B, double* scal, int32_t* state) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= B || !state[2 * i]) return;
-  double* s = scal + i * kS;
-  s[3] = s[6];
-  if (s[3] < s[1]) {
-    state[2 * i] = 0;
-    return;
-  }
-  const double abs_old = s[2];
-  s[2] = s[7];
-  s[5] = s[2] / abs_old;
-  if (++state[2 * i + 1] >= kCgMaxIters) state[2 * i] = 0;
-}
-
 // p = inv * r + beta p
 __global__ __launch_bounds__(kVB) void k_cg_dir(int64_t n, int K, const int32_t* inst, const int32_t* state,
                                                 const double* scal, const double* inv, const double* r, double* p) {
@@ -263,6 +243,121 @@ __global__ __launch_bounds__(kVB) void k_cg_dir(int64_t n, int K, const int32_t*
   if (!state[2 * i]) return;
   const double z = inv[q] * r[q];
   p[q] = z + scal[i * kS + 5] * p[q];
+}
+
+// The two reductions of an iteration, a workgroup per chunk: the products of a
+// chunk are formed with all loads in flight, kept in LDS, added by 256 threads
+// in the order of k_cg_dot (16 each, then its tree), and the last chunk of an
+// instance to finish adds the chunks in order and moves the instance's scalars
+// on.  (An iteration was seven launches beside the product, 30 us of serial
+// loads; now three, 17 us.  One workgroup per instance for all of it: 25 us,
+// bound by one compute unit's loads.)
+constexpr int kCgThreads = 1024, kCgPer = kChunk / kCgThreads;
+
+// sum over the chunk of prod[0 .. kChunk) in LDS; valid in thread 0
+__device__ __forceinline__ double chunk_sum(const double* prod, double* red) {
+  __syncthreads();
+  if (threadIdx.x < kVB) {
+    double a = 0.;
+#pragma unroll
+    for (int m = 0; m < kChunk / kVB; ++m) a += prod[threadIdx.x + m * kVB];
+    red[threadIdx.x] = a;
+  }
+  __syncthreads();
+  double v = 0.;
+  if (threadIdx.x < 64) {
+    const double* s = red + threadIdx.x;
+    v = (s[0] + s[128]) + (s[64] + s[192]);
+    for (int w = 32; w > 0; w /= 2) v += __shfl_down(v, w);
+  }
+  return v;
+}
+
+// Publishes a chunk's sums and tells whether it is its instance's last chunk to
+// do so (thread 0 only).  No chunk waits for another.
+__device__ __forceinline__ bool chunk_done(double* part, double a, double b, int32_t* done, int nchunk) {
+  __hip_atomic_store(&part[2 * blockIdx.x], a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(&part[2 * blockIdx.x + 1], b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __threadfence();
+  if (__hip_atomic_fetch_add(done, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1 < nchunk) return false;
+  __hip_atomic_store(done, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __threadfence();
+  return true;
+}
+__device__ __forceinline__ double chunk_part(const double* part, int c, int w) {
+  return __hip_atomic_load(&part[2 * c + w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// scal[6] = p . t of every instance
+__global__ __launch_bounds__(kCgThreads) void k_cg_pt(const int64_t* chunk, const int32_t* chunk_inst,
+                                                      const int32_t* inst_chunk, const int32_t* state, const double* p,
+                                                      const double* t, double* part, int32_t* done, double* scal) {
+  __shared__ double prod[kChunk], red[kVB];
+  const int i = chunk_inst[blockIdx.x];
+  if (!state[2 * i]) return;
+  const int64_t lo = chunk[2 * blockIdx.x];
+  const int len = static_cast<int>(chunk[2 * blockIdx.x + 1] - lo);
+#pragma unroll
+  for (int m = 0; m < kCgPer; ++m) {
+    const int q = threadIdx.x + m * kCgThreads;
+    prod[q] = q < len ? p[lo + q] * t[lo + q] : 0.;
+  }
+  const double a = chunk_sum(prod, red);
+  if (threadIdx.x) return;
+  const int c0 = inst_chunk[i], c1 = inst_chunk[i + 1];
+  if (!chunk_done(part, a, 0., &done[i], c1 - c0)) return;
+  double s = 0.;
+  for (int c = c0; c < c1; ++c) s += chunk_part(part, c, 0);
+  scal[i * kS + 6] = s;
+}
+
+// x += alpha p, r -= alpha t with alpha = absNew / p.t, then |r|^2 and
+// r.(inv r): converged, or beta and the next absNew (k_cg_update, k_cg_step)
+__global__ __launch_bounds__(kCgThreads) void k_cg_xr(const int64_t* chunk, const int32_t* chunk_inst,
+                                                      const int32_t* inst_chunk, int32_t* state, const double* p,
+                                                      const double* t, const double* inv, double* x, double* r,
+                                                      double* part, int32_t* done, double* scal) {
+  __shared__ double prod[kChunk], red[kVB];
+  const int i = chunk_inst[blockIdx.x];
+  if (!state[2 * i]) return;
+  double* s = scal + i * kS;
+  const double alpha = s[2] / s[6];
+  const int64_t lo = chunk[2 * blockIdx.x];
+  const int len = static_cast<int>(chunk[2 * blockIdx.x + 1] - lo);
+  double rv[kCgPer], iv[kCgPer];
+#pragma unroll
+  for (int m = 0; m < kCgPer; ++m) {
+    const int q = threadIdx.x + m * kCgThreads;
+    rv[m] = iv[m] = 0.;
+    if (q < len) {
+      x[lo + q] += alpha * p[lo + q];
+      rv[m] = r[lo + q] - alpha * t[lo + q];
+      iv[m] = inv[lo + q];
+      r[lo + q] = rv[m];
+    }
+    prod[q] = rv[m] * rv[m];
+  }
+  const double a = chunk_sum(prod, red);
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < kCgPer; ++m) prod[threadIdx.x + m * kCgThreads] = rv[m] * (iv[m] * rv[m]);
+  const double b = chunk_sum(prod, red);
+  if (threadIdx.x) return;
+  const int c0 = inst_chunk[i], c1 = inst_chunk[i + 1];
+  if (!chunk_done(part, a, b, &done[i], c1 - c0)) return;
+  double rr = 0., rz = 0.;
+  for (int c = c0; c < c1; ++c) {
+    rr += chunk_part(part, c, 0);
+    rz += chunk_part(part, c, 1);
+  }
+  s[3] = rr;
+  if (rr < s[1]) {
+    state[2 * i] = 0;
+    return;
+  }
+  s[5] = rz / s[2];
+  s[2] = rz;
+  if (++state[2 * i + 1] >= kCgMaxIters) state[2 * i] = 0;
 }
 
 // right-hand sides of the implicit solves and the final combination
@@ -482,8 +577,8 @@ void Context::visc_operator_apply(const double* x, double* y, int mode, double c
     hipLaunchKernelGGL(k_vop_spmv, dim3(vblocks(n)), dim3(kVB), 0, stream, n, K, vop_rowptr.p, vop_col.p, vop_val.p,
                        x, y, mode, c);
   else
-    hipLaunchKernelGGL(k_vop_spmv_wide, dim3(static_cast<unsigned>(n)), dim3(kWB), 0, stream, K, vop_rowptr.p,
-                       vop_col.p, vop_val.p, x, y, mode, c);
+    hipLaunchKernelGGL(k_vop_spmv_wide, dim3(static_cast<unsigned>((E() + kXcds - 1) / kXcds * kXcds * K)), dim3(kWB), 0,
+                       stream, E(), K, vop_rowptr.p, vop_col.p, vop_val.p, x, y, mode, c);
 }
 
 void Context::rhs_visc_operator() {
@@ -508,17 +603,20 @@ void Context::imex43_init(double dt) {
   }
   // reduction chunks: fixed pieces of each instance's DoF range
   std::vector<int64_t> chunk;
-  std::vector<int32_t> inst_chunk{0};
+  std::vector<int32_t> inst_chunk{0}, chunk_inst;
   for (int i = 0; i < B(); ++i) {
     for (int64_t lo = off[i] * K; lo < off[i + 1] * K; lo += kChunk) {
       chunk.push_back(lo);
       chunk.push_back(std::min<int64_t>(lo + kChunk, off[i + 1] * K));
+      chunk_inst.push_back(i);
     }
     inst_chunk.push_back(static_cast<int32_t>(chunk.size() / 2));
   }
   cg_nchunk = static_cast<int>(chunk.size() / 2);
   to_dev(cg_chunk, chunk, stream);
   to_dev(cg_inst_chunk, inst_chunk, stream);
+  to_dev(cg_chunk_inst, chunk_inst, stream);
+  to_dev(cg_done, std::vector<int32_t>(B(), 0), stream);
   cg_part.ensure(std::max(2 * cg_nchunk, 1));
   cg_scal.ensure(static_cast<size_t>(B()) * kS);
   cg_state.ensure(static_cast<size_t>(B()) * 2);
@@ -532,15 +630,10 @@ int Context::cg_solve(double c) {
   const int64_t n = E() * K;
   const int nB = B();
   if (n == 0) return 0;
-  auto dots = [&](const double* a, const double* b, int mode) {
-    if (cg_nchunk > 0)
-      hipLaunchKernelGGL(k_cg_dot, dim3(cg_nchunk), dim3(kVB), 0, stream, cg_chunk.p, a, b, cg_inv.p, mode,
-                         cg_part.p);
-    hipLaunchKernelGGL(k_cg_sum, dim3((nB + 63) / 64), dim3(64), 0, stream, nB, cg_inst_chunk.p, cg_part.p,
-                       cg_scal.p);
-  };
   hipLaunchKernelGGL(k_cg_start, dim3(vblocks(n)), dim3(kVB), 0, stream, n, cg_b.p, cg_inv.p, u.p, cg_r.p, cg_p.p);
-  dots(cg_r.p, nullptr, 1);
+  if (cg_nchunk > 0)
+    hipLaunchKernelGGL(k_cg_dot, dim3(cg_nchunk), dim3(kVB), 0, stream, cg_chunk.p, cg_r.p, cg_inv.p, cg_part.p);
+  hipLaunchKernelGGL(k_cg_sum, dim3((nB + 63) / 64), dim3(64), 0, stream, nB, cg_inst_chunk.p, cg_part.p, cg_scal.p);
   hipLaunchKernelGGL(k_cg_begin, dim3((nB + 63) / 64), dim3(64), 0, stream, nB, cg_scal.p, cg_state.p);
   std::vector<int32_t> state(2 * nB);
   // The flags are read every kCheck iterations: an instance that converged
@@ -558,11 +651,11 @@ int Context::cg_solve(double c) {
       if (!any) break;
     }
     visc_operator_apply(cg_p.p, cg_t.p, 2, c);
-    dots(cg_p.p, cg_t.p, 0);
-    hipLaunchKernelGGL(k_cg_update, dim3(vblocks(n)), dim3(kVB), 0, stream, n, K, g_inst.p, cg_state.p, cg_scal.p,
-                       cg_p.p, cg_t.p, u.p, cg_r.p);
-    dots(cg_r.p, nullptr, 1);
-    hipLaunchKernelGGL(k_cg_step, dim3((nB + 63) / 64), dim3(64), 0, stream, nB, cg_scal.p, cg_state.p);
+    hipLaunchKernelGGL(k_cg_pt, dim3(cg_nchunk), dim3(kCgThreads), 0, stream, cg_chunk.p, cg_chunk_inst.p,
+                       cg_inst_chunk.p, cg_state.p, cg_p.p, cg_t.p, cg_part.p, cg_done.p, cg_scal.p);
+    hipLaunchKernelGGL(k_cg_xr, dim3(cg_nchunk), dim3(kCgThreads), 0, stream, cg_chunk.p, cg_chunk_inst.p,
+                       cg_inst_chunk.p, cg_state.p, cg_p.p, cg_t.p, cg_inv.p, u.p, cg_r.p, cg_part.p, cg_done.p,
+                       cg_scal.p);
     hipLaunchKernelGGL(k_cg_dir, dim3(vblocks(n)), dim3(kVB), 0, stream, n, K, g_inst.p, cg_state.p, cg_scal.p,
                        cg_inv.p, cg_r.p, cg_p.p);
   }

@@ -56,7 +56,7 @@ __global__ void k_list_zero(int32_t* p, int n) {
 // cell at a time, a thread per (list, target): 590 us for 237 thousand elements
 // of the rotating wave at level 9 (the coarse targets' walks), 168 us for 90 to
 // 165 thousand of 512 Burgers solves, 68 us for 145 elements; a thread per
-// target over words 747, 54 and 24 us; now 118, 29 and 11 us.
+// target over words 747, 54 and 24 us; now 249, 53 and 13 us.
 constexpr int kPiece = 16;
 
 template <int G>
