@@ -161,9 +161,12 @@ Context::ListPlan& Context::get_list_plan(ListForm form) {
   std::vector<Out> outs;                        // output buffers, addressed once the size is known
   std::vector<std::pair<size_t, size_t>> ins;   // inputs that are phase buffers
   std::vector<size_t> rofs_of;                  // per term: first entry of its offsets
-  auto rest_offsets = [&](const int* sin, const int* sout, int dd) {
+  // per rest index (row-major over the dimensions other than dd): offsets in
+  // tensors of input sizes sin with the given strides
+  auto rest_offsets = [&](const int* sin, const int* stin, const int* stout, int dd) {
     std::vector<int> id(sin, sin + D);
-    id.insert(id.end(), sout, sout + D);
+    id.insert(id.end(), stin, stin + D);
+    id.insert(id.end(), stout, stout + D);
     id.push_back(dd);
     auto it = rofs_at.find(id);
     if (it != rofs_at.end()) return it->second;
@@ -172,24 +175,34 @@ Context::ListPlan& Context::get_list_plan(ListForm form) {
     int R = 1;
     for (int d = 0; d < D; ++d) R *= d == dd ? 1 : sin[d];
     for (int r = 0; r < R; ++r) {
-      int rem = r, bi = 0, bo = 0, si = 1, so = 1;
+      int rem = r, bi = 0, bo = 0;
       for (int d = D - 1; d >= 0; --d) {
-        if (d != dd) {
-          const int q = rem % sin[d];
-          rem /= sin[d];
-          bi += q * si;
-          bo += q * so;
-        }
-        si *= sin[d];
-        so *= sout[d];
+        if (d == dd) continue;
+        bi += rem % sin[d] * stin[d];
+        bo += rem % sin[d] * stout[d];
+        rem /= sin[d];
       }
       rofs.push_back(int2{bi, bo});
     }
     return at;
   };
-  // a term over lists of `kind`; sizes before and after the sweep of dd
-  auto make_term = [&](int kind, const double* in, const float* in32, int comp, const int* sin, const int* sout, int dd,
-                       const double* M, int lu, double coef, bool split) {
+  // strides of a tensor of sizes sz: row-major, with dimension `inner` (if not
+  // -1) moved to the innermost place
+  auto strides = [&](const int* sz, int inner, int* st) {
+    int n = 1;
+    if (inner >= 0) {
+      st[inner] = 1;
+      n = sz[inner];
+    }
+    for (int d = D - 1; d >= 0; --d) {
+      if (d == inner) continue;
+      st[d] = n;
+      n *= sz[d];
+    }
+  };
+  // a term over lists of `kind`; sizes and strides before and after the sweep of dd
+  auto make_term = [&](int kind, const double* in, const float* in32, int comp, const int* sin, const int* stin,
+                       const int* sout, const int* stout, int dd, const double* M, int lu, double coef, bool split) {
     ListTerm t{};
     t.in = in; t.in32 = in32; t.M = M; t.ns = 1 << nmax; t.lu = lu; t.coef = coef;
     if (split) {
@@ -204,9 +217,9 @@ Context::ListPlan& Context::get_list_plan(ListForm form) {
     t.Tin = prod_of(sin, D);
     t.Tout = prod_of(sout, D);
     t.R = t.Tin / sin[dd];
-    t.sdd = t.sod = 1;
-    for (int d = dd + 1; d < D; ++d) { t.sdd *= sin[d]; t.sod *= sout[d]; }
-    rofs_of.push_back(rest_offsets(sin, sout, dd));
+    t.sdd = stin[dd];
+    t.sod = stout[dd];
+    rofs_of.push_back(rest_offsets(sin, stin, stout, dd));
     return t;
   };
   auto in_bytes = [&](const ListTerm& t, bool phase_in) { return (phase_in || t.in32 || !f32) ? w : 8.0; };
@@ -236,7 +249,16 @@ Context::ListPlan& Context::get_list_plan(ListForm form) {
         std::vector<double>& v = coefs[prefix(c, st)];
         if (std::find(v.begin(), v.end(), c.coef) == v.end()) v.push_back(c.coef);
       }
-    struct Node { size_t at; bool applied; };  // output of a node; the coefficient is in it
+    // the dimension most of a node's continuations sweep next (the later one on
+    // a tie): innermost in its output, so that they read their values as one run
+    std::map<std::vector<uintptr_t>, std::vector<int>> nexts;
+    for (const Chain& c : chains)
+      for (int st = 0; st + 1 < D; ++st) {
+        std::vector<int>& v = nexts[prefix(c, st)];
+        v.resize(D, 0);
+        ++v[dims[c.o][st + 1]];
+      }
+    struct Node { size_t at; bool applied; int st[kMaxDim]; };  // output of a node; the coefficient is in it
     std::map<std::vector<uintptr_t>, Node> nodes;
     tmp_used = 0;
     phases.clear();
@@ -254,12 +276,23 @@ Context::ListPlan& Context::get_list_plan(ListForm form) {
         const Node* before = st ? &nodes.at(prefix(c, st - 1)) : nullptr;
         const bool applied = before && before->applied;
         const bool here = !applied && (st + 1 == D || coefs[id].size() == 1);
+        int stin[kMaxDim], inner = -1;
+        if (before) std::copy(before->st, before->st + D, stin);
+        else strides(sin, -1, stin);
+        if (st + 1 < D) {
+          const std::vector<int>& v = nexts[id];
+          inner = D - 1;
+          for (int d = D - 1; d >= 0; --d)
+            if (v[d] > v[inner]) inner = d;
+        }
+        Node node{tmp_used, applied || here, {}};
+        strides(sout, inner, node.st);
         ListTerm t = make_term(c.kind[dd], before ? nullptr : c.in, before ? nullptr : c.in32, before ? 0 : c.comp, sin,
-                               sout, dd, c.tab[dd], lus[c.o][st], here ? c.coef : 1.0, f32);
+                               stin, sout, node.st, dd, c.tab[dd], lus[c.o][st], here ? c.coef : 1.0, f32);
         if (before) ins.push_back({flat.size(), before->at});
         ph.bytes += in_bytes(t, before != nullptr) * t.Tin;
         if (st + 1 < D) {
-          nodes[id] = {tmp_used, applied || here};
+          nodes[id] = node;
           outs.push_back({flat.size(), tmp_used});
           tmp_used += t.Tout;
           ph.bytes += w * t.Tout;
@@ -311,9 +344,11 @@ Context::ListPlan& Context::get_list_plan(ListForm form) {
   pl.pen = static_cast<int>(flat.size());
   // the LF penalty stays FP64 in every precision
   int ksz[kMaxDim];
+  int kst[kMaxDim];
   for (int d = 0; d < D; ++d) ksz[d] = k + 1;
+  strides(ksz, -1, kst);
   for (int d = 0; d < D; ++d) {
-    flat.push_back(make_term(LIST_FLX, nullptr, nullptr, 0, ksz, ksz, d, t_aa[4].p, LU_FULL, 0., false));
+    flat.push_back(make_term(LIST_FLX, nullptr, nullptr, 0, ksz, kst, ksz, kst, d, t_aa[4].p, LU_FULL, 0., false));
     if (pen_coef) flat.back().coef_inst = pen_coef + static_cast<size_t>(d) * B();
   }
   list_tmp.ensure(std::max<size_t>(tmp_most * list_ecap, 1));
