@@ -9,6 +9,7 @@
 
 #include <algorithm>
 #include <array>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <atomic>
@@ -276,6 +277,94 @@ __global__ __launch_bounds__(kBlock) void k_flux_herm(const T* up, T* fp, int64_
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_surplus(SurplusArgs a) {
   surplus_point<T>(a, static_cast<int64_t>(xcd_block()) * blockDim.x + threadIdx.x);
+}
+
+// The same, a thread per line of P1 points along the dimension: the cell's
+// ancestors and its P1 x P1 weights are read once for the points and components
+// of a line (a thread per point read them for each, after 64-bit divisions).
+// Bound: the vector memory unit and 16 bytes a value from HBM: 256 3D
+// instances, 213 thousand elements, three components, 195 us a dimension
+// (a thread per point 432).
+template <class T, int P1>
+__global__ __launch_bounds__(kBlock) void k_surplus_line(SurplusArgs a, uint32_t R) {
+  const uint32_t i = xcd_block() * kBlock + threadIdx.x;
+  const uint32_t e = i / R, r = i - e * R;
+  if (e >= a.E) return;
+  const uint32_t sd = a.stride_d, hi = r / sd;
+  const uint32_t own = e * a.P + (hi * P1) * sd + (r - hi * sd);  // first point of the line
+  const uint32_t line = own - e * a.P;
+  const int s = a.slot[e];
+  const T* in = surplus_in<T>(a);
+  T* out;
+  if constexpr (sizeof(T) == 8) out = a.out;
+  else out = a.out32;
+  if (s == 0) {
+    for (int c = 0; c < a.ncomp; ++c)
+#pragma unroll
+      for (int p = 0; p < P1; ++p) out[c * a.comp_stride + own + p * sd] = in[c * a.comp_stride + own + p * sd];
+    return;
+  }
+  const int fb = a.fbase[e];
+  int anc[P1];
+  uint32_t from[P1];
+  bool hole = false;
+#pragma unroll
+  for (int q = 0; q < P1; ++q) {
+    anc[q] = a.fmap[fb + a.anc_slot[s * P1 + q]];
+    from[q] = static_cast<uint32_t>(max(anc[q], 0)) * a.P + line + a.anc_point[s * P1 + q] * sd;
+    hole = hole || anc[q] < 0;
+  }
+  if (hole) atomicOr(a.err, ERR_ANCESTOR);
+  T w[P1 * P1], wl[sizeof(T) == 8 ? 1 : P1 * P1];
+#pragma unroll
+  for (int q = 0; q < P1 * P1; ++q) {
+    if constexpr (sizeof(T) == 8) {
+      w[q] = a.wt[s * (P1 * P1) + q];
+    } else {
+      w[q] = a.wh[s * (P1 * P1) + q];
+      wl[q] = a.wl[s * (P1 * P1) + q];
+    }
+  }
+  for (int c = 0; c < a.ncomp; ++c) {
+    const T* ic = in + c * a.comp_stride;
+    T v[P1], x[P1];
+#pragma unroll
+    for (int p = 0; p < P1; ++p) v[p] = ic[own + p * sd];
+#pragma unroll
+    for (int q = 0; q < P1; ++q) x[q] = ic[from[q]];
+#pragma unroll
+    for (int q = 0; q < P1; ++q) {
+      if (hole && anc[q] < 0) continue;
+#pragma unroll
+      for (int p = 0; p < P1; ++p) {
+        if constexpr (sizeof(T) == 8) {
+          v[p] += w[p * P1 + q] * x[q];
+        } else {
+          v[p] = fmaf(wl[p * P1 + q], x[q], v[p]);
+          v[p] = fmaf(w[p * P1 + q], x[q], v[p]);
+        }
+      }
+    }
+    T* oc = out + c * a.comp_stride;
+#pragma unroll
+    for (int p = 0; p < P1; ++p) oc[own + p * sd] = v[p];
+  }
+}
+
+template <class T>
+void launch_surplus(const SurplusArgs& a, hipStream_t s) {
+  const int64_t n = a.E * a.P;
+  // (32-bit offsets within a component; degree 5 keeps a thread per point)
+  if (a.p1 <= 5 && n < INT_MAX) {
+    const uint32_t R = a.P / a.p1;
+    const dim3 grid(nblocks(a.E * R)), block(kBlock);
+    if (a.p1 == 2) hipLaunchKernelGGL((k_surplus_line<T, 2>), grid, block, 0, s, a, R);
+    else if (a.p1 == 3) hipLaunchKernelGGL((k_surplus_line<T, 3>), grid, block, 0, s, a, R);
+    else if (a.p1 == 4) hipLaunchKernelGGL((k_surplus_line<T, 4>), grid, block, 0, s, a, R);
+    else hipLaunchKernelGGL((k_surplus_line<T, 5>), grid, block, 0, s, a, R);
+    return;
+  }
+  hipLaunchKernelGGL(k_surplus<T>, dim3(nblocks(n * a.ncomp)), dim3(kBlock), 0, s, a);
 }
 
 // One RK stage update (rk_combine); a non-finite result raises ERR_NONFINITE.
@@ -1022,7 +1111,7 @@ void Context::surplus_transform(const double* in, double* out, double* sa, doubl
     a.E = E(); a.comp_stride = E() * P; a.P = P; a.p1 = p1; a.stride_d = stride; a.ncomp = ncomp;
     if (E() > 0) {
       prof_begin(PROF_SURPLUS, 8.0 * static_cast<double>(E()) * P * ncomp * 2);
-      hipLaunchKernelGGL(k_surplus<double>, dim3(nblocks(E() * P * ncomp)), dim3(kBlock), 0, stream, a);
+      launch_surplus<double>(a, stream);
       prof_end();
     }
     cur = dst;
@@ -1044,7 +1133,7 @@ void Context::surplus_transform32(const float* in, float* out, float* sa, float*
     a.E = E(); a.comp_stride = E() * P; a.P = P; a.p1 = p1; a.stride_d = stride; a.ncomp = ncomp;
     if (E() > 0) {
       prof_begin(PROF_SURPLUS, 4.0 * static_cast<double>(E()) * P * ncomp * 2);
-      hipLaunchKernelGGL(k_surplus<float>, dim3(nblocks(E() * P * ncomp)), dim3(kBlock), 0, stream, a);
+      launch_surplus<float>(a, stream);
       prof_end();
     }
     cur = dst;
