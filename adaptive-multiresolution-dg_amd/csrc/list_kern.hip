@@ -15,6 +15,13 @@ constexpr int kWave = 64;
 
 inline unsigned nblocks(int64_t n) { return static_cast<unsigned>((n + kBlock - 1) / kBlock); }
 
+// Sources requested together: four on small grids, where a launch waits for
+// the longest lists of its few wavefronts, two on large ones, where the
+// registers of four cost more resident wavefronts than the overlap saves
+// (4D sparse grid of 10,496 elements: 9.3 ms a run with two, 8.0 with four;
+// 512 2D instances, 90 to 165 thousand elements: 18.9 and 20.0 ms).
+constexpr int64_t kFewElements = 16384;
+
 // ---------------------------------------------------------------------------
 // build
 
@@ -461,7 +468,7 @@ __global__ __launch_bounds__(kBlock) void k_list_phase(const ListTerm* terms, ui
 // value, and the point flux.  A block holds EB elements; each of its
 // wavefronts takes every W-th term for all of them.
 template <int PF, int PT, class T, int NB>
-__global__ __launch_bounds__(512) void k_list_up_final(const ListTerm* terms, int nterm, int EB, int nch, int64_t E,
+__global__ __launch_bounds__(NB == 4 ? 1024 : 512) void k_list_up_final(const ListTerm* terms, int nterm, int EB, int nch, int64_t E,
                                                         int P, const double* u, T* up, T* fp, const double* vcoef,
                                                         int kind, double s, int ncomp) {
   extern __shared__ double vals[];  // [nterm][EB][P]
@@ -491,7 +498,7 @@ __global__ __launch_bounds__(512) void k_list_up_final(const ListTerm* terms, in
 // Last sweep of every right-hand-side partial sum and the penalty sweeps,
 // added in order, then the RK stage update.  Blocks as above.
 template <int PFM, int PFK, class T, int NB>
-__global__ __launch_bounds__(512) void k_list_rhs_final(const ListTerm* terms, int nterm, int npen, int EB, int nch,
+__global__ __launch_bounds__(NB == 4 ? 1024 : 512) void k_list_rhs_final(const ListTerm* terms, int nterm, int npen, int EB, int nch,
                                                         int64_t E, int K, ListRhs a) {
   extern __shared__ double vals[];  // [nterm + npen][EB][K]
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), W = blockDim.x / kWave;
@@ -533,15 +540,15 @@ inline FinalShape final_shape(int nt, int nch, int outs, int64_t E) {
   if (fit < 1) throw std::runtime_error("final kernel: block too large");
   int eb = std::max(1, std::min(kWave / std::min(nch, kWave), fit));
   eb = static_cast<int>(std::min<int64_t>(eb, std::max<int64_t>(E, 1)));
-  return {eb, std::min(nt, 8)};
+  // up to eight wavefronts with equally many terms each (27 terms of three
+  // dimensions on 7, 10 of two on 5: 1740 and 795 us on eight, 1655 and 772 so;
+  // ten wavefronts leave a compute unit fewer blocks: 1883 and 833); sixteen on
+  // small grids, whose time is the terms in turn of the block with the longest
+  // lists (4D, 68 terms: 407 us with eight, 171 with sixteen)
+  const int most = E <= kFewElements ? 16 : 8;
+  const int rounds = (nt + most - 1) / most;
+  return {eb, (nt + rounds - 1) / rounds};
 }
-
-// Sources requested together: four on small grids, where a launch waits for
-// the longest lists of its few wavefronts, two on large ones, where the
-// registers of four cost more resident wavefronts than the overlap saves
-// (4D sparse grid of 10,496 elements: 9.3 ms a run with two, 8.0 with four;
-// 512 2D instances, 90 to 165 thousand elements: 18.9 and 20.0 ms).
-constexpr int64_t kFewElements = 16384;
 
 template <int PF, int PT, class T>
 void phase_t(const ListTerm* terms, int ntask, int64_t E, int R, const double* u, hipStream_t s) {
