@@ -532,6 +532,104 @@ __global__ __launch_bounds__(kAB) void k_ad_run_levels(const int32_t* svals, con
   }
 }
 
+// The fiber tables of a small grid in one launch, a workgroup per dimension:
+// the fiber keys are sorted in LDS, their runs numbered by a prefix sum, and
+// fiber ids, levels and counts written as the launches of the general path do.
+// Bound: latency of the sorting network's barriers, against seven or more
+// launches a dimension of the general path.  A two-dimensional solve of ten
+// steps (twenty grid changes, this and one launch less a remapped field):
+// 7.27 ms -> 5.66 at 168 elements, 8.18 -> 6.57 at 1,033, 8.42 -> 7.03 at
+// 1,520, 8.41 -> 7.71 at 1,993: the gain ends soon after 2,048, where the sort
+// would also need more than 64 KB of LDS at the next power of two.
+constexpr int kSmallFib = 2048, kSmallThreads = 1024;
+struct SmallFibArgs {
+  const int32_t* slot[kMaxDim];
+  const int32_t* inst;
+  int32_t* fbase[kMaxDim];
+  int32_t* fmaxl[kMaxDim];
+  int32_t* lmax;    // [B * D], zeroed
+  int32_t* nfib;    // [D]
+  int32_t* maxfib;  // [D]
+  int N, D, nmax;
+};
+
+__global__ __launch_bounds__(kSmallThreads) void k_ad_fibers_small(SmallFibArgs a) {
+  __shared__ uint64_t key[kSmallFib];
+  __shared__ int32_t val[kSmallFib], top[kSmallFib], len[kSmallFib];
+  __shared__ int32_t wsum[kSmallThreads / 64], most;
+  const int dd = blockIdx.x, tid = threadIdx.x, N = a.N;
+  int n2 = 2;
+  while (n2 < N) n2 <<= 1;
+  for (int q = tid; q < n2; q += kSmallThreads) {
+    uint64_t k = ~uint64_t{0};
+    if (q < N) {
+      k = static_cast<uint64_t>(a.inst[q]) << (a.D * a.nmax);
+      for (int d = 0; d < a.D; ++d)
+        if (d != dd) k |= static_cast<uint64_t>(a.slot[d][q]) << (a.nmax * d);
+    }
+    key[q] = k;
+    val[q] = q;
+    top[q] = len[q] = 0;
+  }
+  if (tid == 0) most = 0;
+  // bitonic sort (elements of one fiber in any order: they share the results)
+  for (int w = 2; w <= n2; w <<= 1)
+    for (int h = w >> 1; h > 0; h >>= 1) {
+      __syncthreads();
+      for (int i = tid; i < n2 / 2; i += kSmallThreads) {
+        const int lo = 2 * i - (i & (h - 1)), hi = lo + h;
+        const uint64_t x = key[lo], y = key[hi];
+        if ((x > y) == ((lo & w) == 0)) {
+          key[lo] = y;
+          key[hi] = x;
+          const int32_t v = val[lo];
+          val[lo] = val[hi];
+          val[hi] = v;
+        }
+      }
+    }
+  __syncthreads();
+  // run numbers: inclusive sum of the run starts, two elements a thread
+  const int q0 = 2 * tid, lane = tid % 64;
+  int s0 = 0, s1 = 0;
+  if (q0 < N) s0 = q0 == 0 || key[q0] != key[q0 - 1];
+  if (q0 + 1 < N) s1 = key[q0 + 1] != key[q0];
+  int inc = s0 + s1;
+  for (int o = 1; o < 64; o <<= 1) {
+    const int v = __shfl_up(inc, o);
+    if (lane >= o) inc += v;
+  }
+  if (lane == 63) wsum[tid / 64] = inc;
+  __syncthreads();
+  int before = 0;
+  for (int w = 0; w < tid / 64; ++w) before += wsum[w];
+  const int run1 = before + inc - 1, run0 = run1 - s1;  // run of q0 + 1, run of q0
+  int32_t e[2] = {0, 0};
+  const int run[2] = {run0, run1};
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+    if (q0 + j < N) {
+      e[j] = val[q0 + j];
+      a.fbase[dd][e[j]] = run[j] << a.nmax;
+      atomicMax(&top[run[j]], slot_level(a.slot[dd][e[j]]));
+      atomicAdd(&len[run[j]], 1);
+      if (q0 + j == N - 1) a.nfib[dd] = run[j] + 1;
+    }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+    if (q0 + j < N) {
+      const int32_t t = top[run[j]];
+      a.fmaxl[dd][e[j]] = t;
+      if (j == 0 ? s0 : s1) {
+        atomicMax(&most, len[run[j]]);
+        atomicMax(a.lmax + a.inst[e[j]] * a.D + dd, t);
+      }
+    }
+  __syncthreads();
+  if (tid == 0) a.maxfib[dd] = most;
+}
+
 // first and last element of every instance in the sorted table
 __global__ __launch_bounds__(kAB) void k_ad_bounds(const int32_t* inst, int64_t N, int32_t* first, int32_t* last) {
   const int64_t q = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -879,6 +977,20 @@ void Context::device_grid_finish(int64_t N, int64_t oldE) {
   int32_t* meta_nfib = meta_lmax + static_cast<int64_t>(B_) * D;
   int32_t* meta_maxfib = meta_nfib + D;
   hipLaunchKernelGGL(k_ad_bounds, dim3(ablocks(N)), dim3(kAB), 0, stream, ad_inst.p, N, ad_meta.p, ad_meta.p + B_);
+  const bool small = N <= kSmallFib;
+  if (small) {
+    SmallFibArgs f{};
+    for (int d = 0; d < D; ++d) {
+      ad_fbase[d].ensure(static_cast<size_t>(std::max<int64_t>(N, 1)));
+      ad_fmaxl[d].ensure(static_cast<size_t>(std::max<int64_t>(N, 1)));
+      f.slot[d] = ad_slot[d].p;
+      f.fbase[d] = ad_fbase[d].p;
+      f.fmaxl[d] = ad_fmaxl[d].p;
+    }
+    f.inst = ad_inst.p; f.lmax = meta_lmax; f.nfib = meta_nfib; f.maxfib = meta_maxfib;
+    f.N = static_cast<int>(N); f.D = D; f.nmax = nmax;
+    hipLaunchKernelGGL(k_ad_fibers_small, dim3(D), dim3(kSmallThreads), 0, stream, f);
+  }
   for (int i = 0; i < 2; ++i) {
     ad_keys[i].ensure(static_cast<size_t>(N));
     ad_vals[i].ensure(static_cast<size_t>(N));
@@ -889,7 +1001,7 @@ void Context::device_grid_finish(int64_t N, int64_t oldE) {
   const int endbit = D * nmax + bits_for(B_);
   size_t cbytes = 0;
   (void)hipcub::DeviceScan::InclusiveSum(nullptr, cbytes, ad_run.p, ad_run.p, static_cast<int>(N), stream);
-  for (int dd = 0; dd < D; ++dd) {
+  for (int dd = 0; dd < D && !small; ++dd) {
     FibArgs f{};
     for (int d = 0; d < D; ++d) f.slot[d] = ad_slot[d].p;
     f.inst = ad_inst.p;

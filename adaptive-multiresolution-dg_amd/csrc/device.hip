@@ -878,14 +878,12 @@ void Context::remap_field(DevBuf<double>& f, int per_elem, const std::vector<int
 }
 
 void Context::remap_field_dev(DevBuf<double>& f, int per_elem, int64_t newE, int64_t old_E) {
-  remap_tmp.ensure(std::max<int64_t>(old_E * per_elem, 1));
-  if (old_E > 0)
-    hipLaunchKernelGGL(k_copy, dim3(nblocks(old_E * per_elem)), dim3(kBlock), 0, stream, remap_tmp.p, f.p,
-                       old_E * per_elem);
-  f.ensure(std::max<int64_t>(newE * per_elem, 1));
+  // into the spare buffer, which then becomes the field
+  remap_tmp.ensure(std::max<int64_t>(newE * per_elem, 1));
   if (newE > 0)
-    hipLaunchKernelGGL(k_remap, dim3(nblocks(newE * per_elem)), dim3(kBlock), 0, stream, f.p, remap_tmp.p,
-                       g_remap.p, newE, per_elem);
+    hipLaunchKernelGGL(k_remap, dim3(nblocks(newE * per_elem)), dim3(kBlock), 0, stream, remap_tmp.p, f.p, g_remap.p,
+                       newE, per_elem);
+  f.swap(remap_tmp);
 }
 
 void Context::set_grid_slots(const std::vector<int32_t>& slots, bool keep_fields) {

@@ -262,3 +262,32 @@ def test_deferred_judge_norm_at_eps_decided_on_host():
     assert sa == sb and pa == pb
     _same(a, b, "eps at a norm")
     assert b.grid_check() == 0
+
+
+@pytest.mark.parametrize("dim,level,batch", [(1, 2, 1), (1, 3, 1), (2, 4, 1), (2, 4, 7), (2, 5, 1), (2, 5, 2), (2, 5, 3),
+                                             (3, 3, 3)])
+def test_fiber_tables_of_small_and_large_tables(dim, level, batch):
+    """Tables of at most 2,048 elements get their fiber tables from one
+    workgroup a dimension, larger ones from a device-wide sort: both against
+    the host build, on full grids of 2^(dim level) elements an instance less
+    some leaves (the coarsened table may be of the small kind where the first
+    one was not)."""
+    print(f"[case] fiber tables dim={dim} level={level} batch={batch}", flush=True)
+    s = pyadg.Solution(dim, 1, 1, level + 1, False, level)
+    s.init_batch(batch, sparse=False, level_init=level)
+    s.set_device_adapt(1)
+    rng = np.random.default_rng(level)
+    full = s.num_elem
+    assert full == batch << (dim * level)
+    u = rng.uniform(0.5, 1.0, (full, s.K))
+    u[rng.choice(full, full // 3, replace=False)] = 0.0
+    s.set(pyadg.FIELD_UCOE, u.reshape(-1))
+    counts = [full]
+    for eps, eta in [(1e30, 1e-3), (1e-12, 1e-13), (0.9, 0.6)]:
+        s.refine(eps)
+        assert s.grid_check() == 0, f"refine {eps}: {s.num_elem} elements"
+        counts.append(s.num_elem)
+        s.coarsen(eta)
+        assert s.grid_check() == 0, f"coarsen {eta}: {s.num_elem} elements"
+        counts.append(s.num_elem)
+    print(f"[device adapt] element counts {counts}", flush=True)

@@ -73,7 +73,8 @@ def test_few_and_many_elements(batch):
     _same(_steps(s, ws[0].problem, -1, 2), _steps(s, ws[0].problem, 3, 2), "adaptive")
 
 
-@pytest.mark.parametrize("dim,k,m,cap", [(1, 1, 2, -1), (2, 3, 3, -1), (3, 2, 3, 3), (4, 1, 2, -1)])
+@pytest.mark.parametrize("dim,k,m,cap", [(1, 1, 2, -1), (2, 3, 3, -1), (3, 2, 3, 3), (4, 1, 2, -1),
+                                         (2, 2, 4, -1), (3, 2, 1, -1)])
 def test_single_operators_match_oracle(dim, k, m, cap):
     """Operators on lists, added to what the right-hand side holds, against
     the oracle; the constant-coefficient operator with both signs of speed."""
