@@ -627,12 +627,8 @@ template <class T>
 void list_phase(int pf1, int pt1, const ListTerm* terms, int ntask, int64_t E, int R, const double* u,
                 hipStream_t s) {
 #define ADG_LP(F, P) if (pf1 == F && pt1 == P) { phase_t<F, P, T>(terms, ntask, E, R, u, s); return; }
-#ifdef ADG_LIST_QUICK
-  ADG_LP(2, 3) ADG_LP(3, 2) ADG_LP(3, 4) ADG_LP(4, 3)
-#else
   ADG_LP(2, 2) ADG_LP(2, 3) ADG_LP(2, 4) ADG_LP(2, 5) ADG_LP(3, 2) ADG_LP(3, 3) ADG_LP(3, 4) ADG_LP(3, 5)
   ADG_LP(4, 2) ADG_LP(4, 3) ADG_LP(4, 4) ADG_LP(4, 5) ADG_LP(5, 2) ADG_LP(5, 3) ADG_LP(5, 4)
-#endif
 #undef ADG_LP
   throw std::runtime_error("list phase: unsupported basis sizes");
 }
@@ -645,12 +641,8 @@ void list_up_final(int k1, int m1, const ListTerm* terms, int nterm, int64_t E, 
     up_final_t<F, Q, T>(terms, nterm, E, P, u, up, fp, vcoef, kind, fs, ncomp, s);        \
     return;                                                                                   \
   }
-#ifdef ADG_LIST_QUICK
-  ADG_LU(2, 3) ADG_LU(3, 4)
-#else
   ADG_LU(2, 2) ADG_LU(2, 3) ADG_LU(2, 4) ADG_LU(2, 5) ADG_LU(3, 2) ADG_LU(3, 3) ADG_LU(3, 4) ADG_LU(3, 5)
   ADG_LU(4, 2) ADG_LU(4, 3) ADG_LU(4, 4) ADG_LU(4, 5)
-#endif
 #undef ADG_LU
   throw std::runtime_error("list up final: unsupported basis sizes");
 }
@@ -663,12 +655,8 @@ void list_rhs_final(int m1, int k1, const ListTerm* terms, int nterm, int npen, 
     rhs_final_t<F, Q, T>(terms, nterm, npen, E, K, r, s);           \
     return;                                                         \
   }
-#ifdef ADG_LIST_QUICK
-  ADG_LR(3, 2) ADG_LR(4, 3)
-#else
   ADG_LR(2, 2) ADG_LR(2, 3) ADG_LR(2, 4) ADG_LR(3, 2) ADG_LR(3, 3) ADG_LR(3, 4) ADG_LR(4, 2) ADG_LR(4, 3)
   ADG_LR(4, 4) ADG_LR(5, 2) ADG_LR(5, 3) ADG_LR(5, 4)
-#endif
 #undef ADG_LR
   throw std::runtime_error("list rhs final: unsupported basis sizes");
 }

@@ -631,7 +631,7 @@ class Solution:
         return st
 
     def set_kernel_variant(self, variant):
-        """Thread mapping of the fused kernels (-1: autotuned)."""
+        """Thread mapping of the fused kernels (-1: source lists)."""
         self._check(lib().adg_set_kernel_variant(self._h, variant))
 
     def set_stage_launch(self, mode):
@@ -648,7 +648,7 @@ class Solution:
         self._check(lib().adg_stage(self._h, ctypes.byref(problem), scheme, stage, dt))
 
     def set_class_variants(self, variants):
-        """Fixed mapping per kernel class (classes 0..3 FP64, 4..7 FP32; -1: autotuner)."""
+        """Fixed mapping per kernel class (classes 0..3 FP64, 4..7 FP32; -1: autotuner; all -1: source lists)."""
         arr = (ctypes.c_int * max(len(variants), 1))(*variants)
         self._check(lib().adg_set_class_variants(self._h, arr, len(variants)))
 

@@ -211,7 +211,7 @@ def main():
                     help="storage precision of the chosen form's fused stages (fp32: split FP32 tables, FP64 "
                          "accumulation, RK and refine/coarsen norms)")
     ap.add_argument("--variant", type=int, default=-1, choices=range(-1, 10),
-                    help="chosen form: thread mapping of every fused kernel (-1: the autotuner picks per class)")
+                    help="chosen form: thread mapping of every fused kernel (-1: sweeps over source lists)")
     ap.add_argument("--mappings", default=None,
                     help="chosen form: thread mapping per fused kernel class (eval-up phases, eval-up final, "
                          "right-hand-side phases, right-hand-side final), e.g. 3,3,7,7; default 'auto': the "

@@ -352,9 +352,12 @@ int adg_set_instance_params(adg_ctx* c, const double* coef_scale, const double* 
  * workgroup stages the inputs of whole fibers in LDS and walks the related
  * cells there, one thread per (element, index over the non-swept dimensions);
  * 7, 8, 9 the same tiles, one thread per element for all those indices.  All
- * mappings give identical results.  -1 (the default) times
- * them on the live grid the first time a kernel meets a grid-size class and
- * keeps the fastest. */
+ * mappings give identical results.  -1 (the default) leaves the mappings
+ * aside: the stages read lists of the related sources of every element, built
+ * once per grid, with the same results.  Where the lists do not fit (k = 3 in
+ * four dimensions, m = 5, lists of more than 4 GiB) or only some classes
+ * are fixed (adg_set_class_variants), the rest is timed on the live grid the
+ * first time a kernel meets a grid-size class and the fastest is kept. */
 int adg_set_kernel_variant(adg_ctx* c, int variant);
 
 /* Artificial viscosity in its matrix-free form (viscosity_option 3 of
@@ -473,7 +476,7 @@ int adg_set_precision(adg_ctx* c, int precision);
 
 /* Launch form of adg_stage and of adg_run_hyperbolic's fused form (no
  * reference counterpart).  0 (default): one launch per phase of the stage
- * (3*dim + up to 3 launches), each with the thread mapping the autotuner or
+ * (3*dim + up to 3 launches), over source lists or with the thread mapping
  * adg_set_kernel_variant picks.  1: one persistent cooperative launch per
  * stage: every workgroup loops over the work items of a phase -- (term, tile
  * of whole fibers) for the sweeps, points for the point flux, the surplus
@@ -505,7 +508,8 @@ int adg_rk_step(adg_ctx* c, const adg_problem* p, int scheme, double dt);
 
 /* Fixed thread mappings per kernel class (no reference counterpart): v[c] for
  * class c = 0..n-1 (n <= 8; classes as in adg_kernel_tuning), -1 leaves the
- * class to the autotuner.  adg_set_kernel_variant, when >= 0, overrides these.
+ * class to the autotuner (all -1: to the source lists).  adg_set_kernel_variant,
+ * when >= 0, overrides these.
  * All mappings give identical values. */
 int adg_set_class_variants(adg_ctx* c, const int* v, int n);
 
