@@ -308,6 +308,7 @@ class Context {
   struct ListPlan;
   std::shared_ptr<ListPlan> list_plans[LIST_FORMS];
   bool list_stage_fits() const;
+  bool stage_on_lists() const;
   ListPlan& get_list_plan(ListForm form);
   template <class T>
   void list_phases(const ListPlan& pl, const std::vector<ListPhase>& phases, int cat, int pf1, int pt1);

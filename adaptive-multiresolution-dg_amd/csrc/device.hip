@@ -1592,6 +1592,14 @@ void Context::tile_launch(int v, int pf1, int pt1, const TaskDev* tasks, int R, 
   tile_sweep<T>(pf1, pt1, tasks, ntask, ts.ntile, ts.max_tile, tb, te, D, lsum_cap, allr, last, stream);
 }
 
+// Whether a fused stage runs on source lists (no mapping of its kernel classes
+// is fixed and the grid is within the list kernels' index ranges).
+bool Context::stage_on_lists() const {
+  bool fixed = kernel_variant >= 0 || stage_launch == 1;
+  for (int c = 0; c < 4; ++c) fixed = fixed || class_variant[c + (precision == 1 ? 4 : 0)] >= 0;
+  return !fixed && list_stage_fits();
+}
+
 void Context::stage_fused(const StageProblem& p, int scheme, int stage, double dt, bool first) {
   if (E() == 0) return;
   if (is_varcoef(p.flux_kind) &&
@@ -1611,9 +1619,7 @@ void Context::stage_fused(const StageProblem& p, int scheme, int stage, double d
     up32.ensure(e * P);
     for (DevBuf<float>* b : {&fp32, &fucoe32, &interA32, &interB32}) b->ensure(e * P * D);
   }
-  bool fixed = kernel_variant >= 0 || stage_launch == 1;
-  for (int c = 0; c < 4; ++c) fixed = fixed || class_variant[c + (precision == 1 ? 4 : 0)] >= 0;
-  if (!fixed && list_stage_fits()) {
+  if (stage_on_lists()) {
     ++stage_count;
     if (precision == 1) stage_list<float>(p, scheme, stage, dt, first);
     else stage_list<double>(p, scheme, stage, dt, first);
@@ -1815,7 +1821,9 @@ void Context::rk_step_eager(const StageProblem& p, int scheme, int nstage, doubl
 // Everything a recorded step depends on besides the contents of device
 // memory: versions of the grid and of the tables built from it, the device
 // buffers (their addresses change when they grow), the problem, the launch
-// settings and, without per-instance steps, dt.
+// settings and, without per-instance steps, dt.  The contents of the source
+// lists follow from the grid, the cap and the family in the key: rk_step()
+// brings the lists up to date before it looks for a recording.
 // positions of the u / u_next addresses in a step key (a step swaps them)
 constexpr size_t kKeyU = 3, kKeyUNext = 4;
 
@@ -1837,7 +1845,7 @@ std::vector<uintptr_t> Context::step_key(const StageProblem& p, int scheme, int 
       static_cast<uintptr_t>(nstage), static_cast<uintptr_t>(p.flux_kind), bits(p.flux_param),
       static_cast<uintptr_t>(use_inst_dt), use_inst_dt ? ptr(d_inst_dt.p) : bits(dt), inst_alpha.size()};
   for (int d = 0; d < D; ++d) key.push_back(bits(p.alpha[d]));
-  for (int64_t v : list_version) key.push_back(static_cast<uintptr_t>(v));
+  for (int v : class_variant) key.push_back(static_cast<uintptr_t>(v + 1));
   key.insert(key.end(), {ptr(list_plans[LIST_STAGE].get()), ptr(list_tmp.p)});
   if (key[kKeyU] != ptr(u.p) || key[kKeyUNext] != ptr(u_next.p)) throw std::logic_error("step key layout");
   return key;
@@ -1859,6 +1867,9 @@ void Context::rk_step(const StageProblem& p, int scheme, int nstage, double dt) 
     rk_step_eager(p, scheme, nstage, dt);
     return;
   }
+  // single operators or steps with another cap or family may have built the
+  // lists since (in the same buffers)
+  if (stage_on_lists()) ensure_lists(LIST_PT, 3);
   const std::vector<uintptr_t> key = step_key(p, scheme, nstage, dt);
   // the key without the u / u_next pair, which every odd step swaps
   auto norm = [](std::vector<uintptr_t> k) {

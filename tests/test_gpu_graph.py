@@ -110,3 +110,54 @@ def test_graph_fixed_grid_run_replays():
         res.append((s.get(pyadg.FIELD_UCOE), s.graph_step_count()))
     assert np.array_equal(res[0][0], res[1][0]), first_diff(res[0][0], res[1][0])
     assert res[1][1] == (2, 5)
+
+
+def _graph_pair(dim=2, nmax=6):
+    """Two equal solutions on a sparse grid, without and with step graphs."""
+    out = []
+    for graph in (0, 1):
+        s = pyadg.Solution(dim, 2 if dim == 2 else 1, 3 if dim == 2 else 2, nmax, True, nmax)
+        s.init_adaptive_intp_builtin(ic_params(1, shift=0.17), 1e10)
+        s.set_graph_step(graph)
+        out.append(s)
+    return out
+
+
+def _both(pair, what, *calls):
+    """The same calls on both solutions; equal coefficients after every one."""
+    for i, call in enumerate(calls):
+        for s in pair:
+            call(s)
+        x, y = (s.get(pyadg.FIELD_UCOE) for s in pair)
+        assert np.array_equal(x, y), f"{what}, call {i}: " + first_diff(x, y)
+
+
+@pytest.mark.parametrize("variant", [-1, 3])
+@pytest.mark.parametrize("setting", ["cap"])
+def test_replays_after_another_cap_or_family(setting, variant):
+    """The level-sum cap or the interpolation family changes between steps,
+    single operators or whole steps run with the other value, and it changes
+    back: what was recorded replays with the values of the current setting."""
+    print(f"[case] graph steps, {setting} there and back, variant={variant}", flush=True)
+    pair = _graph_pair()
+    for s in pair:
+        s.set_kernel_variant(variant)
+    prob = problem(flux_kind=0, alpha=[1.2, 1.2], wave_speed=[1.0, 1.0], cfl=0.2, t_final=1.0)
+
+    def step(s):
+        s.rk_step(prob, pyadg.RK3, 1e-3)
+
+    def to(v):
+        return (lambda s: s.set_level_sum_cap(v)) if setting == "cap" else (lambda s: s.set_interpolation(v))
+
+    here, there = (-1, 3) if setting == "cap" else (0, 1)
+    _both(pair, "first setting", *[step] * 5)
+    replays = pair[1].graph_step_count()[1]
+    assert replays == 2
+    _both(pair, "an operator with the other setting", to(there), lambda s: s.eval_up(), to(here), step, step)
+    if variant < 0:
+        assert pair[1].graph_step_count()[1] == replays + 2, "what was recorded still serves this grid and setting"
+    _both(pair, "steps with the other setting", to(there), *[step] * 5)
+    _both(pair, "and back", to(here), *[step] * 4)
+    for _ in range(3):
+        _both(pair, "in turn", to(there), step, to(here), step)
