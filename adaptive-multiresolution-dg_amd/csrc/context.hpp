@@ -298,6 +298,7 @@ class Context {
   // first: u^n <- u before the stage
   void stage_fused(const StageProblem& p, int scheme, int stage, double dt, bool first = false);
   struct FusedPlan;
+  int64_t plan_serial = 0;  // builds of plans so far; a build's number is never given again
   FusedPlan& fused_plan(const StageProblem& p);
   template <class T>
   void stage_body(const StageProblem& p, FusedPlan& pl, int scheme, int stage, double dt);
@@ -310,6 +311,7 @@ class Context {
   bool list_stage_fits() const;
   bool stage_on_lists() const;
   ListPlan& get_list_plan(ListForm form);
+  int64_t list_stage_serial() const;  // serial number of the stage's plan, 0 without one
   template <class T>
   void list_phases(const ListPlan& pl, const std::vector<ListPhase>& phases, int cat, int pf1, int pt1);
   // alpha: LF constants of the penalty terms (null: their coefficients are 1)

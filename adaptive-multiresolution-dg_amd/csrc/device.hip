@@ -700,6 +700,7 @@ void Context::set_interpolation(int family) {
 }
 
 struct Context::FusedPlan {
+  int64_t serial = 0;  // of this build (Context::plan_serial)
   int64_t version = -1;
   int interp = -1;
   int precision = -1;
@@ -1312,6 +1313,7 @@ Context::FusedPlan& Context::fused_plan(const StageProblem& p) {
   tile_pv.ensure(Ee * K * D);
   if (!plans[slot]) plans[slot].reset(new FusedPlan());
   FusedPlan& pl = *plans[slot];
+  pl.serial = ++plan_serial;
   pl.version = grid_version;
   pl.interp = interp;
   pl.precision = precision;
@@ -1820,7 +1822,9 @@ void Context::rk_step_eager(const StageProblem& p, int scheme, int nstage, doubl
 
 // Everything a recorded step depends on besides the contents of device
 // memory: versions of the grid and of the tables built from it, the device
-// buffers (their addresses change when they grow), the problem, the launch
+// buffers (their addresses change when they grow), the plans that hold their
+// descriptors (by serial number: a plan may be freed or built again in place,
+// and another may come to lie at its address), the problem, the launch
 // settings and, without per-instance steps, dt.  The contents of the source
 // lists follow from the grid, the cap and the family in the key: rk_step()
 // brings the lists up to date before it looks for a recording.
@@ -1839,14 +1843,15 @@ std::vector<uintptr_t> Context::step_key(const StageProblem& p, int scheme, int 
       static_cast<uintptr_t>(order_version), ptr(u.p), ptr(u_next.p), ptr(tn.p), ptr(rhs.p), ptr(up.p), ptr(fp.p),
       ptr(fucoe.p), ptr(interA.p), ptr(interB.p), ptr(fused_tmp.p), ptr(tile_tv.p), ptr(tile_pv.p), ptr(vcoef.p),
       ptr(err_flag.p), ptr(g_inst.p), ptr(d_pen_coef.p), ptr(up32.p), ptr(fp32.p), ptr(fucoe32.p), ptr(interA32.p),
-      ptr(interB32.p), ptr(plans[0].get()), ptr(plans[1].get()), static_cast<uintptr_t>(precision),
+      ptr(interB32.p), static_cast<uintptr_t>(plans[0] ? plans[0]->serial : 0),
+      static_cast<uintptr_t>(plans[1] ? plans[1]->serial : 0), static_cast<uintptr_t>(list_stage_serial()),
+      ptr(list_tmp.p), static_cast<uintptr_t>(precision),
       static_cast<uintptr_t>(interp), static_cast<uintptr_t>(stage_launch), static_cast<uintptr_t>(kernel_variant + 1),
       static_cast<uintptr_t>(lsum_cap), static_cast<uintptr_t>(E()), tuned.size(), static_cast<uintptr_t>(scheme),
       static_cast<uintptr_t>(nstage), static_cast<uintptr_t>(p.flux_kind), bits(p.flux_param),
       static_cast<uintptr_t>(use_inst_dt), use_inst_dt ? ptr(d_inst_dt.p) : bits(dt), inst_alpha.size()};
   for (int d = 0; d < D; ++d) key.push_back(bits(p.alpha[d]));
   for (int v : class_variant) key.push_back(static_cast<uintptr_t>(v + 1));
-  key.insert(key.end(), {ptr(list_plans[LIST_STAGE].get()), ptr(list_tmp.p)});
   if (key[kKeyU] != ptr(u.p) || key[kKeyUNext] != ptr(u_next.p)) throw std::logic_error("step key layout");
   return key;
 }

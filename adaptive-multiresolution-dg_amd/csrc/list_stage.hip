@@ -35,6 +35,7 @@ struct Context::ListPhase {
   double bytes = 0.;  // algorithmic bytes per element
 };
 struct Context::ListPlan {
+  int64_t serial = 0;  // of this build (Context::plan_serial)
   std::vector<uintptr_t> key;
   DevBuf<ListTerm> terms;
   DevBuf<int2> rofs;
@@ -43,6 +44,10 @@ struct Context::ListPlan {
   Phase up_final, rhs_final, flx_final;
   int pen = 0;  // the D penalty sweeps (after rhs_final's terms in the stage's plan)
 };
+
+int64_t Context::list_stage_serial() const {
+  return list_plans[LIST_STAGE] ? list_plans[LIST_STAGE]->serial : 0;
+}
 
 bool Context::list_stage_fits() const {
   if (E() == 0) return false;
@@ -153,6 +158,7 @@ Context::ListPlan& Context::get_list_plan(ListForm form) {
   const double w = f32 ? 4.0 : 8.0;
   list_plan.reset(new ListPlan());
   ListPlan& pl = *list_plan;
+  pl.serial = ++plan_serial;
   std::vector<ListTerm> flat;
   std::vector<int2> rofs;
   std::map<std::vector<int>, size_t> rofs_at;

@@ -133,7 +133,7 @@ def _both(pair, what, *calls):
 
 
 @pytest.mark.parametrize("variant", [-1, 3])
-@pytest.mark.parametrize("setting", ["cap"])
+@pytest.mark.parametrize("setting", ["cap", "family"])
 def test_replays_after_another_cap_or_family(setting, variant):
     """The level-sum cap or the interpolation family changes between steps,
     single operators or whole steps run with the other value, and it changes
@@ -161,3 +161,33 @@ def test_replays_after_another_cap_or_family(setting, variant):
     _both(pair, "and back", to(here), *[step] * 4)
     for _ in range(3):
         _both(pair, "in turn", to(there), step, to(here), step)
+
+
+@pytest.mark.parametrize("variant", [-1, 3])
+def test_replays_after_another_flux_or_precision(variant):
+    """Another flux or precision in between builds other plans: what was
+    recorded on a plan that is gone is not replayed."""
+    print(f"[case] graph steps, flux and precision there and back, variant={variant}", flush=True)
+    pair = _graph_pair()
+    for s in pair:
+        s.set_kernel_variant(variant)
+    kw = dict(alpha=[1.2, 1.2], wave_speed=[1.0, 1.0], cfl=0.2, t_final=1.0)
+    burgers, sincos = problem(flux_kind=0, **kw), problem(flux_kind=1, flux_param=0.7, **kw)
+
+    def step(p):
+        return lambda s: s.rk_step(p, pyadg.RK3, 1e-3)
+
+    _both(pair, "Burgers", *[step(burgers)] * 4)
+    assert pair[1].graph_step_count()[1] > 0
+    for _ in range(3):
+        _both(pair, "the other flux and back", *[step(sincos)] * 3, *[step(burgers)] * 3)
+    for _ in range(3):
+        for s in pair:
+            s.set_precision(pyadg.PREC_FP32_SPLIT)
+        _both(pair, "FP32", *[step(burgers)] * 3)
+        for s in pair:
+            s.set_precision(pyadg.PREC_FP64)
+        _both(pair, "FP64 again", *[step(burgers)] * 3)
+    replays = pair[1].graph_step_count()[1]
+    _both(pair, "Burgers", *[step(burgers)] * 4)
+    assert pair[1].graph_step_count()[1] > replays
