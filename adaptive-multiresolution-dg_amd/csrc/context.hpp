@@ -295,6 +295,7 @@ class Context {
     double flux_param = 0.;
     double alpha[kMaxDim] = {0, 0, 0, 0};
   };
+  void prepare_stage(const StageProblem& p);
   // first: u^n <- u before the stage
   void stage_fused(const StageProblem& p, int scheme, int stage, double dt, bool first = false);
   struct FusedPlan;

@@ -1602,8 +1602,9 @@ bool Context::stage_on_lists() const {
   return !fixed && list_stage_fits();
 }
 
-void Context::stage_fused(const StageProblem& p, int scheme, int stage, double dt, bool first) {
-  if (E() == 0) return;
+// What a stage needs besides its plan, for this problem, grid and settings:
+// flux state, samples of a variable coefficient, FP32 buffers, source lists.
+void Context::prepare_stage(const StageProblem& p) {
   if (is_varcoef(p.flux_kind) &&
       (flux_kind != p.flux_kind || flux_param != p.flux_param || vcoef_version != grid_version)) {
     flux_kind = p.flux_kind;
@@ -1621,6 +1622,12 @@ void Context::stage_fused(const StageProblem& p, int scheme, int stage, double d
     up32.ensure(e * P);
     for (DevBuf<float>* b : {&fp32, &fucoe32, &interA32, &interB32}) b->ensure(e * P * D);
   }
+  if (stage_on_lists()) ensure_lists(LIST_PT, 3);
+}
+
+void Context::stage_fused(const StageProblem& p, int scheme, int stage, double dt, bool first) {
+  if (E() == 0) return;
+  prepare_stage(p);
   if (stage_on_lists()) {
     ++stage_count;
     if (precision == 1) stage_list<float>(p, scheme, stage, dt, first);
@@ -1826,8 +1833,9 @@ void Context::rk_step_eager(const StageProblem& p, int scheme, int nstage, doubl
 // descriptors (by serial number: a plan may be freed or built again in place,
 // and another may come to lie at its address), the problem, the launch
 // settings and, without per-instance steps, dt.  The contents of the source
-// lists follow from the grid, the cap and the family in the key: rk_step()
-// brings the lists up to date before it looks for a recording.
+// lists and the samples of a variable coefficient follow from the grid, the
+// cap, the family and the problem in the key: rk_step() brings them up to date
+// before it looks for a recording.
 // positions of the u / u_next addresses in a step key (a step swaps them)
 constexpr size_t kKeyU = 3, kKeyUNext = 4;
 
@@ -1872,9 +1880,10 @@ void Context::rk_step(const StageProblem& p, int scheme, int nstage, double dt) 
     rk_step_eager(p, scheme, nstage, dt);
     return;
   }
-  // single operators or steps with another cap or family may have built the
-  // lists since (in the same buffers)
-  if (stage_on_lists()) ensure_lists(LIST_PT, 3);
+  // single operators or steps with another cap, family or coefficient may have
+  // built the lists or sampled the coefficient since (in the same buffers), and
+  // the operators after the step take its flux
+  prepare_stage(p);
   const std::vector<uintptr_t> key = step_key(p, scheme, nstage, dt);
   // the key without the u / u_next pair, which every odd step swaps
   auto norm = [](std::vector<uintptr_t> k) {

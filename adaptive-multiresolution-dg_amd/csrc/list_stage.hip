@@ -383,7 +383,6 @@ void Context::list_phases(const ListPlan& pl, const std::vector<ListPhase>& phas
 
 template <class T>
 void Context::stage_list(const StageProblem& p, int scheme, int stage, double dt, bool first) {
-  ensure_lists(LIST_PT, 3);
   ListPlan& pl = get_list_plan(LIST_STAGE);
   constexpr bool f32 = sizeof(T) == 4;
   const int up_kind = interp == 1 ? -1 : p.flux_kind;

@@ -191,3 +191,33 @@ def test_replays_after_another_flux_or_precision(variant):
     replays = pair[1].graph_step_count()[1]
     _both(pair, "Burgers", *[step(burgers)] * 4)
     assert pair[1].graph_step_count()[1] > replays
+
+
+@pytest.mark.parametrize("variant", [-1, 3])
+def test_replays_after_another_coefficient(variant):
+    """The samples of a variable coefficient are made again for another
+    strength or by the flux operator; a step that was recorded with the first
+    strength replays with samples of that strength."""
+    print(f"[case] graph steps, coefficient there and back, variant={variant}", flush=True)
+    pair = _graph_pair(dim=3, nmax=4)
+    for s in pair:
+        s.set_kernel_variant(variant)
+    kw = dict(flux_kind=pyadg.FLUX_VARCOEF, alpha=[1.5] * 3, wave_speed=[1.0] * 3, cfl=0.2, t_final=1.0)
+    weak, strong = problem(flux_param=0.2, **kw), problem(flux_param=0.5, **kw)
+
+    def step(p):
+        return lambda s: s.rk_step(p, pyadg.RK3, 1e-3)
+
+    _both(pair, "first strength", *[step(weak)] * 5)
+    replays = pair[1].graph_step_count()[1]
+    assert replays > 0
+    _both(pair, "the other strength and back", step(strong), *[step(weak)] * 3)
+    _both(pair, "the flux operator in between", lambda s: s.eval_up(), lambda s: s.flux(pyadg.FLUX_VARCOEF, [0.5]),
+          step(weak), step(weak))
+    # the operators after a replayed step take its flux
+    for s in pair:
+        s.flux(pyadg.FLUX_BURGERS)
+    _both(pair, "the operators after a replay", step(weak), lambda s: (s.rhs_zero(), s.rhs_lagr_vol()))
+    x, y = (s.get(pyadg.FIELD_RHS) for s in pair)
+    assert np.array_equal(x, y), first_diff(x, y)
+    assert pair[1].graph_step_count()[1] > replays
