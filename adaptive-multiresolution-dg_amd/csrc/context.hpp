@@ -54,10 +54,11 @@ struct DevBuf {
   }
   void ensure(size_t n) {
     if (n <= cap) return;
-    if (p) hip_check(hipFree(p), "hipFree");
-    p = nullptr;
     size_t c = cap ? cap : 1024;
     while (c < n) c *= 2;
+    if (p) hip_check(hipFree(p), "hipFree");
+    p = nullptr;
+    cap = 0;  // (also when the allocation fails)
     hip_check(hipMalloc(&p, c * sizeof(T)), "hipMalloc");
     cap = c;
   }
