@@ -52,10 +52,14 @@ struct DevBuf {
     std::swap(p, o.p);
     std::swap(cap, o.cap);
   }
-  void ensure(size_t n) {
-    if (n <= cap) return;
+  size_t grown(size_t n) const {  // capacity after ensure(n)
     size_t c = cap ? cap : 1024;
     while (c < n) c *= 2;
+    return c;
+  }
+  void ensure(size_t n) {
+    if (n <= cap) return;
+    const size_t c = grown(n);
     if (p) hip_check(hipFree(p), "hipFree");
     p = nullptr;
     cap = 0;  // (also when the allocation fails)
@@ -306,13 +310,17 @@ class Context {
   void stage_body(const StageProblem& p, FusedPlan& pl, int scheme, int stage, double dt);
   // The stage on source lists (list.hpp), the form that runs unless the caller
   // fixed a mapping for one of its kernel classes: list_stage.hip.
-  enum ListForm { LIST_STAGE = 0, LIST_OPS, LIST_LINEAR, LIST_FORMS };
+  // LIST_OPS_SAME: the right-hand side where all flux components are equal
+  enum ListForm { LIST_STAGE = 0, LIST_UP, LIST_OPS, LIST_OPS_SAME, LIST_PENALTY, LIST_LINEAR, LIST_FORMS };
   struct ListPhase;
   struct ListPlan;
+  struct ListTerms;
   std::shared_ptr<ListPlan> list_plans[LIST_FORMS];
   bool list_stage_fits() const;
   bool stage_on_lists() const;
   ListPlan& get_list_plan(ListForm form);
+  void list_terms(ListForm form, ListPlan& pl, ListTerms& b);
+  int64_t list_places() const;
   int64_t list_stage_serial() const;  // serial number of the stage's plan, 0 without one
   template <class T>
   void list_phases(const ListPlan& pl, const std::vector<ListPhase>& phases, int cat, int pf1, int pt1);
@@ -323,7 +331,8 @@ class Context {
   void stage_list(const StageProblem& p, int scheme, int stage, double dt, bool first);
   // eval_up, rhs_lagr, rhs_penalty and rhs_linear on lists where they fit
   // (the single operators of the C-ABI; the plain form keeps one launch per sweep)
-  bool list_ops_fit() const;
+  bool list_ops_fit(ListForm form, int kind0, int nkind);
+  int64_t list_values[LIST_FORMS] = {-1, -1, -1, -1, -1, -1};  // of the phase buffers, per element
   void eval_up_op();
   void rhs_lagr_op(bool flux_term);
   void rhs_penalty_op(const double* alpha);
@@ -336,6 +345,9 @@ class Context {
   // lists of the given kinds for the current grid, level-sum cap and
   // interpolation family
   void ensure_lists(int kind0, int nkind);
+  bool lists_current(int kind0, int nkind) const;
+  int64_t list_room(int kind, int lmax) const;
+  int deepest_level(int d) const;
   void list_nonzero_tables();
   static constexpr int kListKinds = 4;
   DevBuf<uint32_t> nz_tab[kListKinds];  // pairs of each kind (list_nonzero)

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <climits>
 #include <map>
 
@@ -34,9 +35,10 @@ struct Context::ListPhase {
   int first = 0, n = 0, R = 0;
   double bytes = 0.;  // algorithmic bytes per element
 };
+using ListKey = std::array<uintptr_t, 12 + 6 * kMaxDim>;
 struct Context::ListPlan {
   int64_t serial = 0;  // of this build (Context::plan_serial)
-  std::vector<uintptr_t> key;
+  ListKey key{};  // the addresses that the terms hold and what they were chosen by
   DevBuf<ListTerm> terms;
   DevBuf<int2> rofs;
   using Phase = ListPhase;
@@ -76,11 +78,29 @@ void Context::list_nonzero_tables() {
   nz_interp = interp;
 }
 
-void Context::ensure_lists(int kind0, int nkind) {
+// Entries of a list of this kind at most.  An element of level l has at most
+// l + 1 related cells at levels up to its own in a nested relation, 2 l + 3 in
+// one that counts touching cells, and as many pairs (less itself) with it as the
+// finer one are in the L parts.
+int64_t Context::list_room(int kind, int lmax) const {
+  return E() * (kind == LIST_FLX || kind == LIST_LIN ? 4 * lmax + 4 : 2 * lmax + 1);
+}
+
+int Context::deepest_level(int d) const {
+  int lmax = 0;
+  for (int i = 0; i < B(); ++i) lmax = std::max(lmax, inst_lmax[static_cast<size_t>(i) * D + d]);
+  return lmax;
+}
+
+bool Context::lists_current(int kind0, int nkind) const {
   bool ok = true;
   for (int q = kind0; q < kind0 + nkind; ++q)
     ok = ok && list_version[q] == grid_version && list_level_cap[q] == lsum_cap && list_interp[q] == interp;
-  if (ok) return;
+  return ok;
+}
+
+void Context::ensure_lists(int kind0, int nkind) {
+  if (lists_current(kind0, nkind)) return;
   not_recording("source lists");
   HostTimer timer(*this, HOST_UPLOAD);
   if (kind0 != LIST_LIN && nz_interp != interp) list_nonzero_tables();
@@ -97,20 +117,14 @@ void Context::ensure_lists(int kind0, int nkind) {
   for (int q = 0; q < LIST_KINDS; ++q) a.nz[q] = nz_tab[q].p;
   l_total.ensure(LIST_KINDS * kMaxDim);
   a.total = l_total.p;
-  // An element of level l has at most l + 1 related cells at levels up to its
-  // own in a nested relation, 2 l + 3 in one that counts touching cells, and
-  // as many pairs (less itself) with it as the finer one are in the L parts.
   int deepest = 0;
   for (int d = 0; d < D; ++d) {
-    int lmax = 0;
-    for (int i = 0; i < B(); ++i) lmax = std::max(lmax, inst_lmax[static_cast<size_t>(i) * D + d]);
+    const int lmax = deepest_level(d);
     deepest = std::max(deepest, lmax);
     for (int q = kind0; q < kind0 + nkind; ++q) {
-      const bool touch = q == LIST_FLX || q == LIST_LIN;
-      const int64_t room = E() * (touch ? 4 * lmax + 4 : 2 * lmax + 1);
       const int l = q * D + d;
       l_meta[l].ensure(static_cast<size_t>(E()));
-      l_ent[l].ensure(static_cast<size_t>(room));
+      l_ent[l].ensure(static_cast<size_t>(list_room(q, lmax)));
       a.meta[l] = l_meta[l].p;
       a.ent[l] = l_ent[l].p;
       a.cap[l] = static_cast<int64_t>(l_ent[l].cap);
@@ -125,48 +139,31 @@ void Context::ensure_lists(int kind0, int nkind) {
   }
 }
 
+// Terms of a plan, with the places in the phase buffers still relative.
+struct Context::ListTerms {
+  std::vector<ListTerm> terms;
+  std::vector<int2> rofs;
+  size_t values = 0;                              // of the phase buffers, per element
+  std::vector<std::pair<size_t, size_t>> outs;    // (term, first value of its output buffer)
+  std::vector<std::pair<size_t, size_t>> ins;     // (term, first value of its input) where that is a phase buffer
+  std::vector<size_t> rofs_of;                    // per term: first entry of its offsets
+};
+
 // form LIST_STAGE: volume and flux terms in one set of phases, in the storage
-// of `precision`; LIST_OPS: as separate operators in FP64.
-Context::ListPlan& Context::get_list_plan(ListForm form) {
-  const bool ops = form == LIST_OPS;
+// of `precision`; the others: separate operators in FP64.
+void Context::list_terms(ListForm form, ListPlan& pl, ListTerms& b) {
+  const bool ops = form != LIST_STAGE, f32 = !ops && precision == 1;
+  const bool same = ops ? form == LIST_OPS_SAME : same_flux;
+  auto ptr = [](const void* q) { return reinterpret_cast<uintptr_t>(q); };
+  const double* pen_coef = inst_alpha.empty() ? nullptr : d_pen_coef.p;
   std::vector<std::vector<int>> lus;
   const std::vector<std::vector<int>> dims = transform_orders(D, lus);
   const int nord = static_cast<int>(dims.size());
-  if (E() > list_ecap) {
-    not_recording("stage buffers");
-    list_ecap = (E() + E() / 4 + 1023) / 1024 * 1024;
-    for (auto& q : list_plans) q.reset();
-  }
-  u_next.ensure(static_cast<size_t>(E()) * K);
-  const bool f32 = !ops && precision == 1;
-  auto ptr = [](const void* q) { return reinterpret_cast<uintptr_t>(q); };
-  const double* pen_coef = inst_alpha.empty() ? nullptr : d_pen_coef.p;
-  std::vector<uintptr_t> key = {static_cast<uintptr_t>(same_flux), static_cast<uintptr_t>(is_varcoef(flux_kind)),
-                                static_cast<uintptr_t>(interp), static_cast<uintptr_t>(f32), ptr(t_pt.p),
-                                ptr(t_la_uv.p), ptr(t_la_uvx.p), ptr(t_la_flx.p), ptr(fucoe.p), ptr(fucoe32.p),
-                                ptr(list_tmp.p), ptr(pen_coef), pen_coef ? static_cast<uintptr_t>(B()) : 0};
-  for (int d = 0; d < D; ++d) {
-    for (int q = LIST_PT; q <= LIST_FLX; ++q) {
-      key.push_back(ptr(l_meta[q * D + d].p));
-      key.push_back(ptr(l_ent[q * D + d].p));
-    }
-  }
-  std::shared_ptr<ListPlan>& list_plan = list_plans[form];
-  if (list_plan && list_plan->key == key) return *list_plan;
-  not_recording("stage plan");
-  HostTimer timer(*this, HOST_PLAN);
   const double w = f32 ? 4.0 : 8.0;
-  list_plan.reset(new ListPlan());
-  ListPlan& pl = *list_plan;
-  pl.serial = ++plan_serial;
-  std::vector<ListTerm> flat;
-  std::vector<int2> rofs;
+  std::vector<ListTerm>& flat = b.terms;
+  std::vector<int2>& rofs = b.rofs;
   std::map<std::vector<int>, size_t> rofs_at;
-  size_t tmp_used = 0, tmp_most = 0;  // values per element of the phase buffers
-  struct Out { size_t term, at; };
-  std::vector<Out> outs;                        // output buffers, addressed once the size is known
-  std::vector<std::pair<size_t, size_t>> ins;   // inputs that are phase buffers
-  std::vector<size_t> rofs_of;                  // per term: first entry of its offsets
+  size_t tmp_used = 0;
   // per rest index (row-major over the dimensions other than dd): offsets in
   // tensors of input sizes sin with the given strides
   auto rest_offsets = [&](const int* sin, const int* stin, const int* stout, int dd) {
@@ -225,7 +222,7 @@ Context::ListPlan& Context::get_list_plan(ListForm form) {
     t.R = t.Tin / sin[dd];
     t.sdd = stin[dd];
     t.sod = stout[dd];
-    rofs_of.push_back(rest_offsets(sin, stin, stout, dd));
+    b.rofs_of.push_back(rest_offsets(sin, stin, stout, dd));
     return t;
   };
   auto in_bytes = [&](const ListTerm& t, bool phase_in) { return (phase_in || t.in32 || !f32) ? w : 8.0; };
@@ -295,11 +292,11 @@ Context::ListPlan& Context::get_list_plan(ListForm form) {
         strides(sout, inner, node.st);
         ListTerm t = make_term(c.kind[dd], before ? nullptr : c.in, before ? nullptr : c.in32, before ? 0 : c.comp, sin,
                                stin, sout, node.st, dd, c.tab[dd], lus[c.o][st], here ? c.coef : 1.0, f32);
-        if (before) ins.push_back({flat.size(), before->at});
+        if (before) b.ins.push_back({flat.size(), before->at});
         ph.bytes += in_bytes(t, before != nullptr) * t.Tin;
         if (st + 1 < D) {
           nodes[id] = node;
-          outs.push_back({flat.size(), tmp_used});
+          b.outs.push_back({flat.size(), tmp_used});
           tmp_used += t.Tout;
           ph.bytes += w * t.Tout;
         }
@@ -310,7 +307,7 @@ Context::ListPlan& Context::get_list_plan(ListForm form) {
       if (st + 1 < D) phases.push_back(ph);
       else last = ph;
     }
-    tmp_most = std::max(tmp_most, tmp_used);
+    b.values = std::max(b.values, tmp_used);
   };
   std::vector<Chain> chains;
   for (int o = 0; o < nord; ++o) {
@@ -325,12 +322,13 @@ Context::ListPlan& Context::get_list_plan(ListForm form) {
   pl.up_final.bytes += w * P * (1 + nc) + (is_varcoef(flux_kind) ? 8.0 * P * nc : 0.);
   chains.clear();
   // in the reference order: volume terms for d = 0..D-1, then flux terms
-  for (int ft = 0; ft < 2; ++ft) {
+  const bool rhs = form == LIST_STAGE || form == LIST_OPS || form == LIST_OPS_SAME;
+  for (int ft = 0; ft < 2 && rhs; ++ft) {
     for (int d = 0; d < D; ++d)
       for (int o = 0; o < nord; ++o) {
         Chain c{};
         c.o = o;
-        c.comp = same_flux ? 0 : d;
+        c.comp = same ? 0 : d;
         c.in = fucoe.p;
         c.in32 = f32 ? fucoe32.p : nullptr;
         c.coef = ft ? 0.5 : 1.0;
@@ -345,8 +343,11 @@ Context::ListPlan& Context::get_list_plan(ListForm form) {
       chains.clear();
     }
   }
-  if (!ops) build(chains, m + 1, k + 1, pl.rhs, pl.rhs_final);
-  pl.rhs_final.bytes += 8.0 * K * (1 + 3 + D);
+  if (form == LIST_STAGE) {
+    build(chains, m + 1, k + 1, pl.rhs, pl.rhs_final);
+    pl.rhs_final.bytes += 8.0 * K * (1 + 3 + D);
+  }
+  if (form != LIST_STAGE && form != LIST_PENALTY) return;
   pl.pen = static_cast<int>(flat.size());
   // the LF penalty stays FP64 in every precision
   int ksz[kMaxDim];
@@ -357,16 +358,63 @@ Context::ListPlan& Context::get_list_plan(ListForm form) {
     flat.push_back(make_term(LIST_FLX, nullptr, nullptr, 0, ksz, kst, ksz, kst, d, t_aa[4].p, LU_FULL, 0., false));
     if (pen_coef) flat.back().coef_inst = pen_coef + static_cast<size_t>(d) * B();
   }
-  list_tmp.ensure(std::max<size_t>(tmp_most * list_ecap, 1));
-  key[10] = ptr(list_tmp.p);
-  upload(pl.rofs, rofs, stream);
-  for (const Out& o : outs) flat[o.term].out = list_tmp.p + o.at * list_ecap;
-  for (const auto& i : ins) {
-    flat[i.first].in = list_tmp.p + i.second * list_ecap;
-    if (f32) flat[i.first].in32 = reinterpret_cast<const float*>(flat[i.first].in);
+}
+
+// Element places of the phase buffers that a grid of this size needs.
+int64_t Context::list_places() const {
+  return E() > list_ecap ? (E() + E() / 4 + 1023) / 1024 * 1024 : list_ecap;
+}
+
+Context::ListPlan& Context::get_list_plan(ListForm form) {
+  if (list_places() > list_ecap) {
+    not_recording("stage buffers");
+    list_ecap = list_places();
+    for (auto& q : list_plans) q.reset();
   }
-  for (size_t i = 0; i < flat.size(); ++i) flat[i].rofs = pl.rofs.p + rofs_of[i];
-  upload(pl.terms, flat, stream);
+  const bool ops = form != LIST_STAGE, f32 = !ops && precision == 1;
+  if (!ops) u_next.ensure(static_cast<size_t>(E()) * K);
+  auto ptr = [](const void* q) { return reinterpret_cast<uintptr_t>(q); };
+  const double* pen_coef = inst_alpha.empty() ? nullptr : d_pen_coef.p;
+  ListKey key{};
+  size_t n = 0;
+  auto add = [&](uintptr_t v) { key[n++] = v; };
+  add(ptr(list_tmp.p));
+  add(static_cast<uintptr_t>(interp));
+  if (!ops) {
+    add(static_cast<uintptr_t>(f32));
+    add(static_cast<uintptr_t>(same_flux));
+    add(static_cast<uintptr_t>(is_varcoef(flux_kind)));
+    add(ptr(fucoe32.p));
+  }
+  if (form != LIST_UP) add(ptr(fucoe.p));
+  if (!ops || form == LIST_PENALTY) {
+    add(ptr(pen_coef));
+    add(pen_coef ? static_cast<uintptr_t>(B()) : 0);
+  }
+  for (int q = form == LIST_STAGE || form == LIST_UP ? LIST_PT : LIST_VOL; q <= (form == LIST_UP ? LIST_PT : LIST_FLX); ++q)
+    for (int d = 0; d < D; ++d) {
+      add(ptr(l_meta[q * D + d].p));
+      add(ptr(l_ent[q * D + d].p));
+    }
+  std::shared_ptr<ListPlan>& list_plan = list_plans[form];
+  if (list_plan && list_plan->key == key) return *list_plan;
+  not_recording("stage plan");
+  HostTimer timer(*this, HOST_PLAN);
+  list_plan.reset(new ListPlan());
+  ListPlan& pl = *list_plan;
+  pl.serial = ++plan_serial;
+  ListTerms b;
+  list_terms(form, pl, b);
+  list_tmp.ensure(std::max<size_t>(b.values * list_ecap, 1));
+  key[0] = ptr(list_tmp.p);
+  upload(pl.rofs, b.rofs, stream);
+  for (const auto& o : b.outs) b.terms[o.first].out = list_tmp.p + o.second * list_ecap;
+  for (const auto& i : b.ins) {
+    b.terms[i.first].in = list_tmp.p + i.second * list_ecap;
+    if (f32) b.terms[i.first].in32 = reinterpret_cast<const float*>(b.terms[i.first].in);
+  }
+  for (size_t i = 0; i < b.terms.size(); ++i) b.terms[i].rofs = pl.rofs.p + b.rofs_of[i];
+  upload(pl.terms, b.terms, stream);
   sync();  // the host vectors are gone after this call
   pl.key = key;
   return pl;
@@ -433,15 +481,50 @@ template void Context::stage_list<float>(const StageProblem&, int, int, double, 
 // 12).  The sums are the same: the sweep-by-sweep form adds term after term to
 // the output as well.
 
-bool Context::list_ops_fit() const {
-  // (Lagrange degree 5 has no list kernels)
-  return m <= 4 && list_stage_fits();
+// The sweep-by-sweep form needs two buffers of an element's values and no
+// lists.  Lists and phase buffers take more (bytes an element with k = 2, m = 3:
+// 1.8 K beside 2.1 K of fields in 2D at level 9, 10 K beside 11 K in 3D at level
+// 7, 108 K beside 52 K in 4D at level 8), so the operators run on lists while
+// these need at most 16 GiB (millions of elements in 2D, one in 3D, a hundred
+// thousand in 4D) and half of the free memory, or where a stage holds them
+// already; beyond, and where the offsets do not fit, sweep by sweep.
+constexpr int64_t kListOpsBytes = int64_t{16} << 30;
+
+bool Context::list_ops_fit(ListForm form, int kind0, int nkind) {
+  // (Lagrange degree 5 has list kernels for the constant-coefficient operator only)
+  if ((m > 4 && form != LIST_LINEAR) || !list_stage_fits()) return false;
+  if (lists_current(kind0, nkind) && (form == LIST_LINEAR || (E() <= list_ecap && list_plans[form]))) return true;
+  int64_t all = 0, more = 0;  // bytes needed, and bytes of them not yet held
+  auto need = [&](auto& buf, int64_t n) {
+    const int64_t item = sizeof(*buf.p), c = static_cast<int64_t>(buf.grown(static_cast<size_t>(n)));
+    all += item * c;
+    if (c > static_cast<int64_t>(buf.cap)) more += item * c;
+  };
+  for (int q = kind0; q < kind0 + nkind; ++q)
+    for (int d = 0; d < D; ++d) {
+      need(l_meta[q * D + d], E());
+      need(l_ent[q * D + d], list_room(q, deepest_level(d)));
+    }
+  if (form != LIST_LINEAR) {
+    if (list_values[form] < 0) {
+      ListPlan pl;
+      ListTerms b;
+      list_terms(form, pl, b);
+      list_values[form] = static_cast<int64_t>(b.values);
+    }
+    need(list_tmp, list_values[form] * list_places());
+  }
+  if (more == 0) return true;
+  if (all > kListOpsBytes) return false;
+  size_t free = 0, total = 0;
+  hip_check(hipMemGetInfo(&free, &total), "hipMemGetInfo");
+  return more <= static_cast<int64_t>(free / 2);
 }
 
 void Context::eval_up_op() {
-  if (!list_ops_fit()) { eval_up(); return; }
-  ensure_lists(LIST_PT, 3);
-  const ListPlan& pl = get_list_plan(LIST_OPS);
+  if (!list_ops_fit(LIST_UP, LIST_PT, 1)) { eval_up(); return; }
+  ensure_lists(LIST_PT, 1);
+  const ListPlan& pl = get_list_plan(LIST_UP);
   list_phases<double>(pl, pl.up, PROF_SWEEP, k + 1, m + 1);
   prof_begin(PROF_SWEEP, pl.up_final.bytes * E());
   list_up_final<double>(k + 1, m + 1, pl.terms.p + pl.up_final.first, pl.up_final.n, E(), P, u.p, up.p, fp.p, vcoef.p, -1,
@@ -450,9 +533,10 @@ void Context::eval_up_op() {
 }
 
 void Context::rhs_lagr_op(bool flux_term) {
-  if (!list_ops_fit()) { rhs_lagr(flux_term); return; }
-  ensure_lists(LIST_PT, 3);
-  const ListPlan& pl = get_list_plan(LIST_OPS);
+  const ListForm form = same_flux ? LIST_OPS_SAME : LIST_OPS;
+  if (!list_ops_fit(form, LIST_VOL, 2)) { rhs_lagr(flux_term); return; }
+  ensure_lists(LIST_VOL, 2);
+  const ListPlan& pl = get_list_plan(form);
   const ListPhase& last = flux_term ? pl.flx_final : pl.rhs_final;
   list_phases<double>(pl, flux_term ? pl.flx : pl.rhs, PROF_RHS_PHASE, m + 1, k + 1);
   ListRhs r = list_rhs(true, 0, 0, 0., false, nullptr);
@@ -463,9 +547,9 @@ void Context::rhs_lagr_op(bool flux_term) {
 }
 
 void Context::rhs_penalty_op(const double* alpha) {
-  if (!list_ops_fit()) { rhs_penalty(alpha); return; }
-  ensure_lists(LIST_PT, 3);
-  const ListPlan& pl = get_list_plan(LIST_OPS);
+  if (!list_ops_fit(LIST_PENALTY, LIST_VOL, 2)) { rhs_penalty(alpha); return; }
+  ensure_lists(LIST_VOL, 2);
+  const ListPlan& pl = get_list_plan(LIST_PENALTY);
   ListRhs r = list_rhs(true, 0, 0, 0., false, alpha);
   r.u_next = nullptr;
   prof_begin(PROF_SWEEP, 8.0 * E() * K * (2 + D));
@@ -479,11 +563,12 @@ void Context::linear_list(const double* coef, bool run, int scheme, int stage, d
   linear_tables(coef);
   ensure_lists(LIST_LIN, 1);
   u_next.ensure(static_cast<size_t>(E()) * K);
-  std::vector<uintptr_t> key = {reinterpret_cast<uintptr_t>(l_meta[LIST_LIN * D].p)};
+  ListKey key{};
+  size_t n = 0;
   for (int d = 0; d < D; ++d)
     for (const void* q : {static_cast<const void*>(l_meta[LIST_LIN * D + d].p), static_cast<const void*>(l_ent[LIST_LIN * D + d].p),
                           static_cast<const void*>(t_lin[d].p)})
-      key.push_back(reinterpret_cast<uintptr_t>(q));
+      key[n++] = reinterpret_cast<uintptr_t>(q);
   std::shared_ptr<ListPlan>& pl = list_plans[LIST_LINEAR];
   if (!pl || pl->key != key) {
     pl.reset(new ListPlan());
@@ -522,7 +607,7 @@ void Context::linear_list(const double* coef, bool run, int scheme, int stage, d
 
 // One RK stage of du/dt = A u; first: u^n <- u before it.
 void Context::linear_stage(const double* coef, int scheme, int stage, double dt, bool first) {
-  if (list_stage_fits()) {
+  if (list_ops_fit(LIST_LINEAR, LIST_LIN, 1)) {
     linear_list(coef, true, scheme, stage, dt, first);
     return;
   }
@@ -533,7 +618,7 @@ void Context::linear_stage(const double* coef, int scheme, int stage, double dt,
 }
 
 void Context::rhs_linear_op(const double* coef) {
-  if (list_stage_fits()) linear_list(coef, false, 0, 0, 0., false);
+  if (list_ops_fit(LIST_LINEAR, LIST_LIN, 1)) linear_list(coef, false, 0, 0, 0., false);
   else rhs_linear(coef);
 }
 

@@ -3,6 +3,8 @@ against the fused per-element kernels and the per-sweep path, bit for bit:
 every basis size the fused stage provides, both interpolation families, the
 level-sum cap, FP32 storage, the single operators, and grids on both sides of the size at which the
 kernels request more sources at a time (16,384 elements)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -103,3 +105,74 @@ def test_single_operators_match_oracle(dim, k, m, cap):
     for field in (pyadg.FIELD_UCOE, pyadg.FIELD_RHS, pyadg.FIELD_TN):
         a, b = g.get(field), o.get(field)
         assert np.array_equal(a, b), f"field {field}: " + first_diff(a, b)
+
+
+def _free_bytes():
+    """Free memory of the device, from the runtime that the library uses."""
+    with open("/proc/self/maps") as f:
+        path = next(line.split()[-1] for line in f if "libamdhip64" in line)
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert ctypes.CDLL(path).hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_operators_of_large_grids_keep_their_memory():
+    """On a grid whose phase buffers would take gigabytes (4D, k = 2, m = 3: 84 KB an element and room
+    to grow) the right-hand side runs sweep by sweep, in buffers that the context has: the same values as on lists."""
+    batch, dim, nmax = 16, 4, 8
+    print(f"[case] operators of a large 4D batch={batch} nmax={nmax}", flush=True)
+
+    def rhs(s):
+        s.eval_up()
+        s.flux(pyadg.FLUX_VARCOEF, [0.3])
+        s.fp_to_coe()
+        s.rhs_zero()
+        s.rhs_lagr_vol()
+        s.rhs_lagr_flx()
+        s.rhs_penalty([1.1] * dim)
+
+    one, many = (pyadg.Solution(dim, 2, 3, nmax, True, nmax) for _ in range(2))
+    many.init_batch(batch)
+    n = one.num_elem * one.K
+    assert many.num_elem == batch * one.num_elem and many.num_elem > 160000
+    u = np.random.default_rng(3).standard_normal(n) * 0.1
+    one.set(pyadg.FIELD_UCOE, u)
+    many.set(pyadg.FIELD_UCOE, np.tile(u, batch))
+    many.sync()
+    before = _free_bytes()
+    rhs(many)
+    many.sync()
+    assert before - _free_bytes() < 12 << 30  # (lists and the phase buffers of the point values)
+    rhs(one)
+    want = one.get(pyadg.FIELD_RHS)
+    for i in range(batch):
+        got = many.instance_get(i, pyadg.FIELD_RHS)
+        assert np.array_equal(got, want), f"instance {i}: " + first_diff(got, want)
+
+
+def test_operators_keep_a_plan_per_flux():
+    """Operators of one flux and then another, again and again: nothing is planned anew (a plan's upload waits for
+    the device), and the values are those of contexts that keep to one flux."""
+    kinds = (pyadg.FLUX_BURGERS, pyadg.FLUX_SINCOS)
+
+    def rhs(s, kind):
+        s.eval_up()
+        s.flux(kind, [0.6])
+        s.fp_to_coe()
+        s.rhs_zero()
+        s.rhs_lagr_vol()
+        s.rhs_lagr_flx()
+        return s.get(pyadg.FIELD_RHS)
+
+    sols = [pyadg.Solution(2, 2, 3, 5, True, 5) for _ in range(3)]
+    for s in sols:
+        s.init_adaptive_intp_builtin(ic_params(1, shift=0.13), 1e10)
+    want = [rhs(sols[i], kinds[i]) for i in range(2)]
+    for i in range(2):
+        rhs(sols[2], kinds[i])
+    sols[2].profile(True)
+    for turn in range(3):
+        for i in range(2):
+            got = rhs(sols[2], kinds[i])
+            assert np.array_equal(got, want[i]), f"turn {turn}, flux {kinds[i]}: " + first_diff(got, want[i])
+    assert sols[2].profile_host()["plan"] == 0.0
