@@ -1605,6 +1605,8 @@ bool Context::stage_on_lists() const {
 // What a stage needs besides its plan, for this problem, grid and settings:
 // flux state, samples of a variable coefficient, FP32 buffers, source lists.
 void Context::prepare_stage(const StageProblem& p) {
+  // (the fused kernels, on lists or by mapping, end at Lagrange degree 4)
+  if (m > 4) throw std::runtime_error("fused stage: unsupported basis sizes (interpolation degree 5 needs the per-sweep form)");
   if (is_varcoef(p.flux_kind) &&
       (flux_kind != p.flux_kind || flux_param != p.flux_param || vcoef_version != grid_version)) {
     flux_kind = p.flux_kind;

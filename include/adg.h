@@ -355,9 +355,11 @@ int adg_set_instance_params(adg_ctx* c, const double* coef_scale, const double* 
  * mappings give identical results.  -1 (the default) leaves the mappings
  * aside: the stages read lists of the related sources of every element, built
  * once per grid, with the same results.  Where the lists do not fit (k = 3 in
- * four dimensions, m = 5, lists of more than 4 GiB) or only some classes
- * are fixed (adg_set_class_variants), the rest is timed on the live grid the
- * first time a kernel meets a grid-size class and the fastest is kept. */
+ * four dimensions, 2^24 elements or more, lists or fields past 4 GiB offsets) or
+ * only some classes are fixed (adg_set_class_variants), the rest is timed on
+ * the live grid the first time a kernel meets a grid-size class and the fastest
+ * is kept.  For m = 5 there are no fused kernels: the fused stages return an
+ * error before any launch, and the single operators run sweep by sweep. */
 int adg_set_kernel_variant(adg_ctx* c, int variant);
 
 /* Artificial viscosity in its matrix-free form (viscosity_option 3 of

@@ -330,3 +330,16 @@ def test_fused_stage_refuses_lagrange_degree_5():
     g.rk_init()
     with pytest.raises(pyadg.AdgError, match="unsupported basis sizes"):
         g.stage(prob, pyadg.RK3, 0, 1e-3)
+
+
+def test_refused_stage_leaves_the_context_usable():
+    # the refusal comes before any launch or timing: the profile can be read, the operators go on
+    g = pyadg.Solution(2, 2, 5, 4, True, 4)
+    prob = problem(flux_kind=0, alpha=[1.2, 1.2], wave_speed=[1.0, 1.0], cfl=0.2, t_final=1.0)
+    g.profile(True)
+    with pytest.raises(pyadg.AdgError, match="unsupported basis sizes"):
+        g.rk_step(prob, pyadg.RK3, 1e-3)
+    assert sum(v["count"] for v in g.profile_get().values()) == 0
+    g.eval_up()
+    assert g.profile_get()["sweep"]["count"] > 0
+    g.profile(False)
