@@ -2007,6 +2007,7 @@ void Context::check_error_flag() {
     hip_check(hipMemcpyAsync(err_flag.p, &z, sizeof(int32_t), hipMemcpyHostToDevice, stream), "upload");
     sync();
     if (h & ERR_ANCESTOR) throw std::runtime_error("surplus transform: missing ancestor element (grid has a hole)");
+    if (h & ERR_LIST) throw std::runtime_error("source lists: more related cells than a grid of these levels has");
     if (h & ERR_COOP) throw std::runtime_error("persistent stage: kernel was not launched cooperatively");
     throw std::runtime_error("RK stage: non-finite value in the solution");
   }

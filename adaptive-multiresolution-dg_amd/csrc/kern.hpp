@@ -144,7 +144,9 @@ __device__ __forceinline__ void flux_point(int kind, T u, double s, const double
 // Error flags of the device (bit values of the context's flag word).
 // ERR_COOP: a persistent stage kernel found itself launched without the
 // cooperative guarantee (it exits at once, leaving the stage undone).
-enum : int32_t { ERR_ANCESTOR = 1, ERR_NONFINITE = 2, ERR_COOP = 4 };
+// ERR_LIST: a source list holds more entries than it has room for (those of
+// the block are left out).
+enum : int32_t { ERR_ANCESTOR = 1, ERR_NONFINITE = 2, ERR_COOP = 4, ERR_LIST = 8 };
 
 // ---- per-element gather kernels (fused_elem.hip): thread mappings 0..3 ----
 // v: 0 thread per output, 1 thread per (element, rest index), 2 thread per

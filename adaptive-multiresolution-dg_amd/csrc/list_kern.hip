@@ -143,7 +143,7 @@ __global__ __launch_bounds__(kBlock) void k_list_build(ListBuildArgs a, int kind
     const int list = (kind0 + q) * a.D + d;
     int at = beg[q] + s_base[q] + s_wave[q][wave], left = n[q];
     if (static_cast<int64_t>(at) + left > a.cap[list]) {  // (the host's bound is exceeded: never)
-      atomicOr(a.err, ERR_COOP);
+      atomicOr(a.err, ERR_LIST);
       left = all[q] = 0;
     }
     if (g == 0) a.meta[list][e] = make_int4(all[q] ? at : 0, all[q] ? nu[q] | all[q] << 16 : 0, st, a.inst[e]);

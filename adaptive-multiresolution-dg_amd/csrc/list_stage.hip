@@ -78,10 +78,10 @@ void Context::list_nonzero_tables() {
   nz_interp = interp;
 }
 
-// Entries of a list of this kind at most.  An element of level l has at most
-// l + 1 related cells at levels up to its own in a nested relation, 2 l + 3 in
+// Room for the entries of a list of this kind.  An element of level l has at most
+// l + 1 related cells at levels up to its own in a nested relation, 2 l + 1 in
 // one that counts touching cells, and as many pairs (less itself) with it as the
-// finer one are in the L parts.
+// finer one are in the L parts: 2 l + 1 and 4 l + 1 entries an element.
 int64_t Context::list_room(int kind, int lmax) const {
   return E() * (kind == LIST_FLX || kind == LIST_LIN ? 4 * lmax + 4 : 2 * lmax + 1);
 }
