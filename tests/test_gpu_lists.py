@@ -1,8 +1,9 @@
 """The stage on source lists (the form that runs when no mapping is fixed)
 against the fused per-element kernels and the per-sweep path, bit for bit:
 every basis size the fused stage provides, both interpolation families, the
-level-sum cap, FP32 storage, the single operators, and grids on both sides of the size at which the
-kernels request more sources at a time (16,384 elements)."""
+level-sum cap, FP32 storage, the single operators, and grids on both sides of
+the size at which the kernels change (16,384 elements): above it two sources are
+in flight instead of four, and the lanes of a target share table blocks."""
 import ctypes
 
 import numpy as np
@@ -73,6 +74,55 @@ def test_few_and_many_elements(batch):
     _same(_steps(s, p, -1, 1), _steps(s, p, 3, 1), "fixed grid")
     # refinement and coarsening grow and shrink the lists
     _same(_steps(s, ws[0].problem, -1, 2), _steps(s, ws[0].problem, 3, 2), "adaptive")
+
+
+def _many(dim, k, m, nmax):
+    """A batch of more than 16,384 elements with coefficients that fall off with the level."""
+    s = pyadg.Solution(dim, k, m, nmax, True, nmax)
+    batch = 16384 // s.num_elem + 2
+    s.init_batch(batch)
+    lev = np.concatenate([s.instance_grid(i)[0] for i in range(batch)])
+    u = np.random.default_rng(dim * 100 + k * 10 + m).standard_normal((len(lev), s.K))
+    s.set(pyadg.FIELD_UCOE, (u * 0.2 * 2.0 ** (-1.5 * lev.sum(axis=1))[:, None]).reshape(-1))
+    assert s.num_elem > 16384
+    return s, batch
+
+
+# phases where the lanes of a target share table blocks: blocks of 4, 6, 9, 12, 16 and 20 values (whole and half
+# 16-byte pieces, single words), one and two pieces a lane, FP32 halves; and the widths that are not shared
+@pytest.mark.parametrize("dim,k,m,nmax,fp32,herm", [
+    (1, 2, 3, 7, 0, 0), (2, 1, 1, 6, 0, 0), (2, 2, 2, 6, 0, 0), (2, 3, 3, 5, 0, 0), (2, 3, 4, 5, 1, 0), (2, 2, 3, 5, 1, 1),
+    (2, 2, 3, 6, 0, 1), (3, 1, 1, 4, 0, 0), (3, 2, 2, 4, 0, 0), (3, 2, 2, 4, 1, 0), (3, 2, 3, 4, 0, 0), (3, 2, 3, 4, 1, 0),
+    (3, 3, 3, 3, 0, 0), (3, 1, 4, 4, 1, 0), (4, 1, 2, 3, 0, 0), (4, 1, 2, 3, 1, 0), (4, 2, 1, 2, 0, 0)])
+def test_many_elements_of_every_block(dim, k, m, nmax, fp32, herm):
+    print(f"[case] lists, many elements dim={dim} k={k} m={m} nmax={nmax} fp32={fp32} herm={herm}", flush=True)
+    s, batch = _many(dim, k, m, nmax)
+    s.set_interpolation(herm)
+    s.set_precision(fp32)
+    s.save_state(0)
+    flux = pyadg.FLUX_BURGERS if dim < 3 else pyadg.FLUX_VARCOEF
+    p = problem(flux_kind=flux, flux_param=0.4, alpha=[1.3] * dim, wave_speed=[1.0] * dim, cfl=0.05, t_final=1.0,
+                adaptive=0, eps=0.0, eta=0.0, max_steps=0, t_start=0.0)
+    got = _steps(s, p, -1, 1)
+    _same(got, _steps(s, p, 1, 1), "per-element kernels")
+    if not fp32:
+        _same(got, _steps(s, p, -1, 1, form=0), "per-sweep path")
+
+
+@pytest.mark.parametrize("dim,cap", [(2, -1), (2, 4), (3, 3)])
+def test_many_elements_with_caps_and_instance_constants(dim, cap):
+    print(f"[case] lists, many elements dim={dim} cap={cap}, constants per instance", flush=True)
+    s, batch = _many(dim, 2, 3, 6 if dim == 2 else 4)
+    s.set_level_sum_cap(cap)
+    s.save_state(0)
+    r = np.random.default_rng(5)
+    s.set_instance_params(coef_scale=r.uniform(0.5, 1.5, (batch, dim)), alpha=r.uniform(0.5, 2.0, (batch, dim)))
+    for flux in (pyadg.FLUX_BURGERS, pyadg.FLUX_VARCOEF_SCALED):
+        p = problem(flux_kind=flux, flux_param=0.4, alpha=[1.3] * dim, wave_speed=[1.0] * dim, cfl=0.05, t_final=1.0,
+                    adaptive=0, eps=0.0, eta=0.0, max_steps=0, t_start=0.0)
+        got = _steps(s, p, -1, 1)
+        _same(got, _steps(s, p, 3, 1), f"flux {flux}, per-element kernels")
+        _same(got, _steps(s, p, -1, 1, form=0), f"flux {flux}, per-sweep path")
 
 
 @pytest.mark.parametrize("dim,k,m,cap", [(1, 1, 2, -1), (2, 3, 3, -1), (3, 2, 3, 3), (4, 1, 2, -1),
