@@ -44,7 +44,7 @@ struct Context::ListPlan {
   using Phase = ListPhase;
   std::vector<Phase> up, rhs, flx;
   Phase up_final, rhs_final, flx_final;
-  int pen = 0;  // the D penalty sweeps (after rhs_final's terms in the stage's plan)
+  int pen = 0;  // the D penalty sweeps (after rhs_final's terms in the stage's plan; not in eval_up's)
 };
 
 int64_t Context::list_stage_serial() const {
@@ -347,7 +347,7 @@ void Context::list_terms(ListForm form, ListPlan& pl, ListTerms& b) {
     build(chains, m + 1, k + 1, pl.rhs, pl.rhs_final);
     pl.rhs_final.bytes += 8.0 * K * (1 + 3 + D);
   }
-  if (form != LIST_STAGE && form != LIST_PENALTY) return;
+  if (form == LIST_UP) return;
   pl.pen = static_cast<int>(flat.size());
   // the LF penalty stays FP64 in every precision
   int ksz[kMaxDim];
@@ -386,8 +386,8 @@ Context::ListPlan& Context::get_list_plan(ListForm form) {
     add(static_cast<uintptr_t>(is_varcoef(flux_kind)));
     add(ptr(fucoe32.p));
   }
-  if (form != LIST_UP) add(ptr(fucoe.p));
-  if (!ops || form == LIST_PENALTY) {
+  add(ptr(fucoe.p));
+  if (form != LIST_UP) {
     add(ptr(pen_coef));
     add(pen_coef ? static_cast<uintptr_t>(B()) : 0);
   }
@@ -489,6 +489,7 @@ template void Context::stage_list<float>(const StageProblem&, int, int, double, 
 // thousand in 4D) and half of the free memory, or where a stage holds them
 // already; beyond, and where the offsets do not fit, sweep by sweep.
 constexpr int64_t kListOpsBytes = int64_t{16} << 30;
+constexpr int64_t kListOpsFree = int64_t{64} << 20;  // taken without a look at the free memory
 
 bool Context::list_ops_fit(ListForm form, int kind0, int nkind) {
   // (Lagrange degree 5 has list kernels for the constant-coefficient operator only)
@@ -500,12 +501,21 @@ bool Context::list_ops_fit(ListForm form, int kind0, int nkind) {
     all += item * c;
     if (c > static_cast<int64_t>(buf.cap)) more += item * c;
   };
-  for (int q = kind0; q < kind0 + nkind; ++q)
-    for (int d = 0; d < D; ++d) {
+  for (int d = 0; d < D; ++d) {
+    const int lmax = deepest_level(d);
+    for (int q = kind0; q < kind0 + nkind; ++q) {
       need(l_meta[q * D + d], E());
-      need(l_ent[q * D + d], list_room(q, deepest_level(d)));
+      need(l_ent[q * D + d], list_room(q, lmax));
     }
+  }
   if (form != LIST_LINEAR) {
+    // every sweep of every chain in a buffer of its own: no plan takes more, and
+    // on small grids that is little enough to count nothing
+    const int64_t nord = D == 1 ? 1 : int64_t{1} << (D - 1), chains = form == LIST_UP ? nord : D * nord;
+    int64_t T = 1;
+    for (int d = 0; d < D; ++d) T *= std::max(k, m) + 1;
+    const int64_t most = form == LIST_PENALTY ? 1 : std::max<int64_t>(chains * (D - 1) * T, 1);
+    if (all + 8 * static_cast<int64_t>(list_tmp.grown(static_cast<size_t>(most * list_places()))) <= kListOpsFree) return true;
     if (list_values[form] < 0) {
       ListPlan pl;
       ListTerms b;
@@ -514,7 +524,7 @@ bool Context::list_ops_fit(ListForm form, int kind0, int nkind) {
     }
     need(list_tmp, list_values[form] * list_places());
   }
-  if (more == 0) return true;
+  if (more == 0 || all <= kListOpsFree) return true;
   if (all > kListOpsBytes) return false;
   size_t free = 0, total = 0;
   hip_check(hipMemGetInfo(&free, &total), "hipMemGetInfo");
@@ -547,9 +557,12 @@ void Context::rhs_lagr_op(bool flux_term) {
 }
 
 void Context::rhs_penalty_op(const double* alpha) {
-  if (!list_ops_fit(LIST_PENALTY, LIST_VOL, 2)) { rhs_penalty(alpha); return; }
+  // the right-hand side's plan holds the sweeps too; without one they need no phase buffers
+  const ListForm rhs_form = same_flux ? LIST_OPS_SAME : LIST_OPS;
+  const ListForm form = list_plans[rhs_form] && E() <= list_ecap ? rhs_form : LIST_PENALTY;
+  if (!list_ops_fit(form, LIST_VOL, 2)) { rhs_penalty(alpha); return; }
   ensure_lists(LIST_VOL, 2);
-  const ListPlan& pl = get_list_plan(LIST_PENALTY);
+  const ListPlan& pl = get_list_plan(form);
   ListRhs r = list_rhs(true, 0, 0, 0., false, alpha);
   r.u_next = nullptr;
   prof_begin(PROF_SWEEP, 8.0 * E() * K * (2 + D));
