@@ -487,7 +487,11 @@ template void Context::stage_list<float>(const StageProblem&, int, int, double, 
 // 7, 108 K beside 52 K in 4D at level 8), so the operators run on lists while
 // these need at most 16 GiB (millions of elements in 2D, one in 3D, a hundred
 // thousand in 4D) and half of the free memory, or where a stage holds them
-// already; beyond, and where the offsets do not fit, sweep by sweep.
+// already; beyond, and where the offsets do not fit, sweep by sweep.  Both sides,
+// a right-hand side by operators: 4D level 8, 168 thousand elements, 82.6 ms sweep
+// by sweep, 49.1 on lists with 32.6 GiB, 74.6 with the point values alone on
+// lists (8.5 GiB); 3D level 7, 109 thousand, 8.3 and 3.1 ms (1.2 GiB); 2D level 9,
+// 180 thousand, 6.8 and 1.7 ms (0.4 GiB).
 constexpr int64_t kListOpsBytes = int64_t{16} << 30;
 constexpr int64_t kListOpsFree = int64_t{64} << 20;  // taken without a look at the free memory
 

@@ -110,7 +110,7 @@ __global__ __launch_bounds__(kPB) void k_features(FeatArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// training: forward and backward thread per sample, gradients thread per parameter
+// training: forward and backward thread per sample, gradients by matrix tiles over chunks of samples
 
 __device__ __forceinline__ float sigmoidf(float z) { return 1.f / (1.f + expf(-z)); }
 

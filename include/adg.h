@@ -498,9 +498,10 @@ int adg_stage_launch_count(adg_ctx* c, int64_t* launches, int64_t* stages);
  * and dt (or the per-instance steps' buffer) -- and replay it from then on.
  * Any change of that state, a grid change by refine or coarsen first of all,
  * makes the next step run without a graph and the one after record a new
- * graph.  Up to four recorded steps are kept.  Results are identical with and
- * without graphs; with profiling on, steps run without graphs.  on = 0 drops
- * the recorded steps. */
+ * graph.  Up to four recorded steps are kept.  Settings and operators between
+ * steps (cap, family, flux, coefficient) may change and change back: a step
+ * replays with what is set.  Results are identical with and without graphs; with
+ * profiling on, steps run without graphs.  on = 0 drops the recorded steps. */
 int adg_set_graph_step(adg_ctx* c, int on);
 /* Steps recorded into graphs and steps replayed from them since creation. */
 int adg_graph_step_count(adg_ctx* c, int64_t* captures, int64_t* replays);
