@@ -318,7 +318,7 @@ class Context {
   std::shared_ptr<ListPlan> list_plans[LIST_FORMS];
   bool list_stage_fits() const;
   bool stage_on_lists() const;
-  ListPlan& get_list_plan(ListForm form);
+  ListPlan& get_list_plan(ListForm form, bool split = false);
   void list_terms(ListForm form, ListPlan& pl, ListTerms& b);
   int64_t list_places() const;
   int64_t list_stage_serial() const;  // serial number of the stage's plan, 0 without one
@@ -331,8 +331,11 @@ class Context {
   void stage_list(const StageProblem& p, int scheme, int stage, double dt, bool first);
   // eval_up, rhs_lagr, rhs_penalty and rhs_linear on lists where they fit
   // (the single operators of the C-ABI; the plain form keeps one launch per sweep)
-  bool list_ops_fit(ListForm form, int kind0, int nkind);
-  int64_t list_values[LIST_FORMS] = {-1, -1, -1, -1, -1, -1};  // of the phase buffers, per element
+  // sweep by sweep, or on lists: all directions at once or one after another
+  enum ListWay { WAY_SWEEPS, WAY_JOINED, WAY_SPLIT };
+  ListWay list_ops_way(ListForm form, int kind0, int nkind);
+  // values of the phase buffers, per element: joined, split (-1: not counted)
+  int64_t list_values[LIST_FORMS][2] = {{-1, -1}, {-1, -1}, {-1, -1}, {-1, -1}, {-1, -1}, {-1, -1}};
   void eval_up_op();
   void rhs_lagr_op(bool flux_term);
   void rhs_penalty_op(const double* alpha);

@@ -35,15 +35,23 @@ struct Context::ListPhase {
   int first = 0, n = 0, R = 0;
   double bytes = 0.;  // algorithmic bytes per element
 };
-using ListKey = std::array<uintptr_t, 12 + 6 * kMaxDim>;
+using ListKey = std::array<uintptr_t, 16 + 6 * kMaxDim>;
 struct Context::ListPlan {
   int64_t serial = 0;  // of this build (Context::plan_serial)
   ListKey key{};  // the addresses that the terms hold and what they were chosen by
   DevBuf<ListTerm> terms;
   DevBuf<int2> rofs;
   using Phase = ListPhase;
-  std::vector<Phase> up, rhs, flx;
-  Phase up_final, rhs_final, flx_final;
+  std::vector<Phase> up, rhs;
+  Phase up_final, rhs_final;
+  // the volume (0) and flux (1) operators: all directions at once, or (split) one
+  // after another in the same phase buffers
+  struct Op {
+    std::vector<Phase> phases;
+    Phase last;
+  };
+  std::vector<Op> ops[2];
+  bool split = false;
   int pen = 0;  // the D penalty sweeps (after rhs_final's terms in the stage's plan; not in eval_up's)
 };
 
@@ -310,21 +318,28 @@ void Context::list_terms(ListForm form, ListPlan& pl, ListTerms& b) {
     b.values = std::max(b.values, tmp_used);
   };
   std::vector<Chain> chains;
-  for (int o = 0; o < nord; ++o) {
-    Chain c{};
-    c.o = o;
-    c.coef = 1.0;
-    for (int d = 0; d < D; ++d) { c.kind[d] = LIST_PT; c.tab[d] = t_pt.p; }
-    chains.push_back(c);
+  if (form == LIST_STAGE || form == LIST_UP) {
+    for (int o = 0; o < nord; ++o) {
+      Chain c{};
+      c.o = o;
+      c.coef = 1.0;
+      for (int d = 0; d < D; ++d) { c.kind[d] = LIST_PT; c.tab[d] = t_pt.p; }
+      chains.push_back(c);
+    }
+    build(chains, k + 1, m + 1, pl.up, pl.up_final);
+    const int nc = ops ? 0 : (same ? 1 : D);
+    pl.up_final.bytes += w * P * (1 + nc) + (is_varcoef(flux_kind) ? 8.0 * P * nc : 0.);
+    chains.clear();
   }
-  build(chains, k + 1, m + 1, pl.up, pl.up_final);
-  const int nc = same_flux ? 1 : D;
-  pl.up_final.bytes += w * P * (1 + nc) + (is_varcoef(flux_kind) ? 8.0 * P * nc : 0.);
-  chains.clear();
   // in the reference order: volume terms for d = 0..D-1, then flux terms
   const bool rhs = form == LIST_STAGE || form == LIST_OPS || form == LIST_OPS_SAME;
+  auto build_op = [&](int ft) {
+    pl.ops[ft].emplace_back();
+    build(chains, m + 1, k + 1, pl.ops[ft].back().phases, pl.ops[ft].back().last);
+    chains.clear();
+  };
   for (int ft = 0; ft < 2 && rhs; ++ft) {
-    for (int d = 0; d < D; ++d)
+    for (int d = 0; d < D; ++d) {
       for (int o = 0; o < nord; ++o) {
         Chain c{};
         c.o = o;
@@ -338,10 +353,9 @@ void Context::list_terms(ListForm form, ListPlan& pl, ListTerms& b) {
         }
         chains.push_back(c);
       }
-    if (ops) {
-      build(chains, m + 1, k + 1, ft ? pl.flx : pl.rhs, ft ? pl.flx_final : pl.rhs_final);
-      chains.clear();
+      if (pl.split) build_op(ft);
     }
+    if (ops && !pl.split) build_op(ft);
   }
   if (form == LIST_STAGE) {
     build(chains, m + 1, k + 1, pl.rhs, pl.rhs_final);
@@ -365,7 +379,7 @@ int64_t Context::list_places() const {
   return E() > list_ecap ? (E() + E() / 4 + 1023) / 1024 * 1024 : list_ecap;
 }
 
-Context::ListPlan& Context::get_list_plan(ListForm form) {
+Context::ListPlan& Context::get_list_plan(ListForm form, bool split) {
   if (list_places() > list_ecap) {
     not_recording("stage buffers");
     list_ecap = list_places();
@@ -380,6 +394,7 @@ Context::ListPlan& Context::get_list_plan(ListForm form) {
   auto add = [&](uintptr_t v) { key[n++] = v; };
   add(ptr(list_tmp.p));
   add(static_cast<uintptr_t>(interp));
+  add(static_cast<uintptr_t>(split));
   if (!ops) {
     add(static_cast<uintptr_t>(f32));
     add(static_cast<uintptr_t>(same_flux));
@@ -403,6 +418,7 @@ Context::ListPlan& Context::get_list_plan(ListForm form) {
   list_plan.reset(new ListPlan());
   ListPlan& pl = *list_plan;
   pl.serial = ++plan_serial;
+  pl.split = split;
   ListTerms b;
   list_terms(form, pl, b);
   list_tmp.ensure(std::max<size_t>(b.values * list_ecap, 1));
@@ -484,26 +500,34 @@ template void Context::stage_list<float>(const StageProblem&, int, int, double, 
 // The sweep-by-sweep form needs two buffers of an element's values and no
 // lists.  Lists and phase buffers take more (bytes an element with k = 2, m = 3:
 // 1.8 K beside 2.1 K of fields in 2D at level 9, 10 K beside 11 K in 3D at level
-// 7, 108 K beside 52 K in 4D at level 8), so the operators run on lists while
-// these need at most 16 GiB (millions of elements in 2D, one in 3D, a hundred
-// thousand in 4D) and half of the free memory, or where a stage holds them
-// already; beyond, and where the offsets do not fit, sweep by sweep.  Both sides,
-// a right-hand side by operators: 4D level 8, 168 thousand elements, 82.6 ms sweep
-// by sweep, 49.1 on lists with 32.6 GiB, 74.6 with the point values alone on
-// lists (8.5 GiB); 3D level 7, 109 thousand, 8.3 and 3.1 ms (1.2 GiB); 2D level 9,
-// 180 thousand, 6.8 and 1.7 ms (0.4 GiB).
-constexpr int64_t kListOpsBytes = int64_t{16} << 30;
+// 7, 108 K beside 52 K in 4D at level 8).  So past 1 GiB of phase buffers the
+// volume and flux operators go direction by direction (4D: 33 K; the launches
+// that this adds are nothing there, and equal fluxes share no sweeps between
+// directions), and the operators run on lists while these need at most 16 GiB
+// and half of the free memory, or where a stage holds them already; beyond, and
+// where the offsets do not fit, sweep by sweep.  A right-hand side by operators:
+// 4D level 8, 168 thousand elements, 82.6 ms sweep by sweep, 49.1 joined with 32.6
+// GiB, 48.4 direction by direction with 8.5 GiB; 3D level 7, 109 thousand, 8.3 and
+// 3.2 ms (1.2 GiB); 2D level 9, 180 thousand, 6.8 and 1.7 ms (0.4 GiB).
+constexpr int64_t kListOpsJoined = int64_t{1} << 30, kListOpsBytes = int64_t{16} << 30;
 constexpr int64_t kListOpsFree = int64_t{64} << 20;  // taken without a look at the free memory
 
-bool Context::list_ops_fit(ListForm form, int kind0, int nkind) {
+Context::ListWay Context::list_ops_way(ListForm form, int kind0, int nkind) {
   // (Lagrange degree 5 has list kernels for the constant-coefficient operator only)
-  if ((m > 4 && form != LIST_LINEAR) || !list_stage_fits()) return false;
-  if (lists_current(kind0, nkind) && (form == LIST_LINEAR || (E() <= list_ecap && list_plans[form]))) return true;
+  if ((m > 4 && form != LIST_LINEAR) || !list_stage_fits()) return WAY_SWEEPS;
+  if (lists_current(kind0, nkind)) {
+    if (form == LIST_LINEAR) return WAY_JOINED;
+    if (list_plans[form] && E() <= list_ecap) return list_plans[form]->split ? WAY_SPLIT : WAY_JOINED;
+  }
+  ListWay way = WAY_JOINED;
   int64_t all = 0, more = 0;  // bytes needed, and bytes of them not yet held
+  auto bytes = [](auto& buf, int64_t n) {
+    return static_cast<int64_t>(sizeof(*buf.p)) * static_cast<int64_t>(buf.grown(static_cast<size_t>(n)));
+  };
+  auto held = [](auto& buf, int64_t n) { return n <= static_cast<int64_t>(buf.cap); };
   auto need = [&](auto& buf, int64_t n) {
-    const int64_t item = sizeof(*buf.p), c = static_cast<int64_t>(buf.grown(static_cast<size_t>(n)));
-    all += item * c;
-    if (c > static_cast<int64_t>(buf.cap)) more += item * c;
+    all += bytes(buf, n);
+    if (!held(buf, n)) more += bytes(buf, n);
   };
   for (int d = 0; d < D; ++d) {
     const int lmax = deepest_level(d);
@@ -512,31 +536,38 @@ bool Context::list_ops_fit(ListForm form, int kind0, int nkind) {
       need(l_ent[q * D + d], list_room(q, lmax));
     }
   }
-  if (form != LIST_LINEAR) {
+  const bool rhs = form == LIST_OPS || form == LIST_OPS_SAME;
+  if (rhs || form == LIST_UP) {
     // every sweep of every chain in a buffer of its own: no plan takes more, and
     // on small grids that is little enough to count nothing
-    const int64_t nord = D == 1 ? 1 : int64_t{1} << (D - 1), chains = form == LIST_UP ? nord : D * nord;
+    const int64_t nord = D == 1 ? 1 : int64_t{1} << (D - 1);
     int64_t T = 1;
     for (int d = 0; d < D; ++d) T *= std::max(k, m) + 1;
-    const int64_t most = form == LIST_PENALTY ? 1 : std::max<int64_t>(chains * (D - 1) * T, 1);
-    if (all + 8 * static_cast<int64_t>(list_tmp.grown(static_cast<size_t>(most * list_places()))) <= kListOpsFree) return true;
-    if (list_values[form] < 0) {
-      ListPlan pl;
-      ListTerms b;
-      list_terms(form, pl, b);
-      list_values[form] = static_cast<int64_t>(b.values);
-    }
-    need(list_tmp, list_values[form] * list_places());
+    const int64_t most = std::max<int64_t>((rhs ? D * nord : nord) * (D - 1) * T, 1);
+    if (all + bytes(list_tmp, most * list_places()) <= kListOpsFree) return way;
+    auto values = [&](bool split) {
+      int64_t& v = list_values[form][split];
+      if (v < 0) {
+        ListPlan pl;
+        pl.split = split;
+        ListTerms b;
+        list_terms(form, pl, b);
+        v = static_cast<int64_t>(b.values);
+      }
+      return v * list_places();
+    };
+    if (rhs && !held(list_tmp, values(false)) && bytes(list_tmp, values(false)) > kListOpsJoined) way = WAY_SPLIT;
+    need(list_tmp, values(way == WAY_SPLIT));
   }
-  if (more == 0 || all <= kListOpsFree) return true;
-  if (all > kListOpsBytes) return false;
+  if (more == 0 || all <= kListOpsFree) return way;
+  if (all > kListOpsBytes) return WAY_SWEEPS;
   size_t free = 0, total = 0;
   hip_check(hipMemGetInfo(&free, &total), "hipMemGetInfo");
-  return more <= static_cast<int64_t>(free / 2);
+  return more <= static_cast<int64_t>(free / 2) ? way : WAY_SWEEPS;
 }
 
 void Context::eval_up_op() {
-  if (!list_ops_fit(LIST_UP, LIST_PT, 1)) { eval_up(); return; }
+  if (list_ops_way(LIST_UP, LIST_PT, 1) == WAY_SWEEPS) { eval_up(); return; }
   ensure_lists(LIST_PT, 1);
   const ListPlan& pl = get_list_plan(LIST_UP);
   list_phases<double>(pl, pl.up, PROF_SWEEP, k + 1, m + 1);
@@ -548,25 +579,28 @@ void Context::eval_up_op() {
 
 void Context::rhs_lagr_op(bool flux_term) {
   const ListForm form = same_flux ? LIST_OPS_SAME : LIST_OPS;
-  if (!list_ops_fit(form, LIST_VOL, 2)) { rhs_lagr(flux_term); return; }
+  const ListWay way = list_ops_way(form, LIST_VOL, 2);
+  if (way == WAY_SWEEPS) { rhs_lagr(flux_term); return; }
   ensure_lists(LIST_VOL, 2);
-  const ListPlan& pl = get_list_plan(form);
-  const ListPhase& last = flux_term ? pl.flx_final : pl.rhs_final;
-  list_phases<double>(pl, flux_term ? pl.flx : pl.rhs, PROF_RHS_PHASE, m + 1, k + 1);
+  const ListPlan& pl = get_list_plan(form, way == WAY_SPLIT);
   ListRhs r = list_rhs(true, 0, 0, 0., false, nullptr);
   r.u_next = nullptr;
-  prof_begin(PROF_SWEEP, last.bytes * E());
-  list_rhs_final<double>(m + 1, k + 1, pl.terms.p + last.first, last.n, 0, E(), K, r, stream);
-  prof_end();
+  for (const ListPlan::Op& op : pl.ops[flux_term]) {
+    list_phases<double>(pl, op.phases, PROF_RHS_PHASE, m + 1, k + 1);
+    prof_begin(PROF_SWEEP, op.last.bytes * E());
+    list_rhs_final<double>(m + 1, k + 1, pl.terms.p + op.last.first, op.last.n, 0, E(), K, r, stream);
+    prof_end();
+  }
 }
 
 void Context::rhs_penalty_op(const double* alpha) {
   // the right-hand side's plan holds the sweeps too; without one they need no phase buffers
   const ListForm rhs_form = same_flux ? LIST_OPS_SAME : LIST_OPS;
   const ListForm form = list_plans[rhs_form] && E() <= list_ecap ? rhs_form : LIST_PENALTY;
-  if (!list_ops_fit(form, LIST_VOL, 2)) { rhs_penalty(alpha); return; }
+  const ListWay way = list_ops_way(form, LIST_VOL, 2);
+  if (way == WAY_SWEEPS) { rhs_penalty(alpha); return; }
   ensure_lists(LIST_VOL, 2);
-  const ListPlan& pl = get_list_plan(form);
+  const ListPlan& pl = get_list_plan(form, way == WAY_SPLIT);
   ListRhs r = list_rhs(true, 0, 0, 0., false, alpha);
   r.u_next = nullptr;
   prof_begin(PROF_SWEEP, 8.0 * E() * K * (2 + D));
@@ -624,7 +658,7 @@ void Context::linear_list(const double* coef, bool run, int scheme, int stage, d
 
 // One RK stage of du/dt = A u; first: u^n <- u before it.
 void Context::linear_stage(const double* coef, int scheme, int stage, double dt, bool first) {
-  if (list_ops_fit(LIST_LINEAR, LIST_LIN, 1)) {
+  if (list_ops_way(LIST_LINEAR, LIST_LIN, 1) != WAY_SWEEPS) {
     linear_list(coef, true, scheme, stage, dt, first);
     return;
   }
@@ -635,7 +669,7 @@ void Context::linear_stage(const double* coef, int scheme, int stage, double dt,
 }
 
 void Context::rhs_linear_op(const double* coef) {
-  if (list_ops_fit(LIST_LINEAR, LIST_LIN, 1)) linear_list(coef, false, 0, 0, 0., false);
+  if (list_ops_way(LIST_LINEAR, LIST_LIN, 1) != WAY_SWEEPS) linear_list(coef, false, 0, 0, 0., false);
   else rhs_linear(coef);
 }
 
